@@ -38,14 +38,16 @@ def listed():
     """The smallest scene of the repository's configurations, its largest, and
     odd sizes between; both precisions; each layer of a step by itself."""
     return [
-        # two stacked cubes, the first configuration: every launch is short,
-        # a pass is latency
-        {"name": "step-two-cubes", "kind": "step", "scene": "pile", "n": 10, "m": 1, "layers": 2,
+        # whole steps of a small slab in FP64: every launch is short, a pass
+        # is latency (steps are taken of slabs only: the 200 to 400 solver
+        # iterations of a stiff pile amplify a last bit into the frame, so
+        # piles are measured by their directions and line searches)
+        {"name": "step-slab-small", "kind": "step", "scene": "slab", "nx": 10, "ny": 16, "nz": 10,
          "fp32": False, "warm": False, "steps": 3},
         # the 1M-tet compressed slab of the benchmark, in its fastest form
         {"name": "step-slab-1m", "kind": "step", "scene": "slab", "nx": 50, "ny": 80, "nz": 50,
          "fp32": True, "warm": True, "steps": 4},
-        # a Newton direction of the smallest scene, every result in FP64
+        # a Newton direction of two stacked cubes, the first configuration
         {"name": "direction-two-cubes", "kind": "direction", "scene": "pile", "n": 10, "m": 1, "layers": 2,
          "fp32": False},
         # an ordinary model of a ragged size
@@ -83,7 +85,7 @@ def draw(rng):
     if kind == "ccd":
         return {"kind": kind, "pairs": log_int(16, 100000), "edges": rng.random() < 0.5}
     case = {"kind": kind}
-    if kind == "predict" or rng.random() < 0.5:
+    if kind in ("step", "predict") or rng.random() < 0.5:
         v = log_int(500, 200000)
         a, b = rng.uniform(0.6, 1.6), rng.uniform(0.6, 1.6)
         nx = max(4, int((v / (a * b)) ** (1 / 3)))
@@ -99,7 +101,7 @@ def draw(rng):
     if kind in ("step", "direction"):
         case["fp32"] = rng.random() < 0.5
     if kind == "step":
-        case |= {"warm": case["fp32"] and case["scene"] == "slab", "steps": rng.randint(1, 3)}
+        case |= {"warm": case["fp32"], "steps": rng.randint(1, 3)}
     return case
 
 
@@ -299,8 +301,8 @@ def _direction(st):
     sim.solve_system(tol=sim.pcg_tol_search)
     if st["case"]["fp32"]:
         sim.refine_solve()
-    return {"counts": np.array(counts), "residual": sim.output_residual(), "rhs": sim.vector(2),
-            "direction": sim.vector(1)}
+    done = sim.output_residual() < sim.setup.newton_tol  # the Newton test
+    return {"counts": np.array(counts), "done": int(done), "rhs": sim.vector(2), "direction": sim.vector(1)}
 
 
 def _linesearch(st):
@@ -398,6 +400,10 @@ def work(case):
 
 
 # ---- the same in 64 bits ----------------------------------------------------
+def _device():
+    return torch.device("cuda" if torch.cuda.is_available() else "cpu")
+
+
 def _exact_mlp(case, seed):
     X, T = (torch.from_numpy(a).double() for a in _rows(case, seed))
     w = torch.from_numpy(_weights().copy()).double().requires_grad_(case["backward"])
@@ -414,40 +420,313 @@ def _exact_mlp(case, seed):
     return {"loss": loss.detach(), "grad": torch.autograd.grad(loss, w)[0]}
 
 
+class _Elastic:
+    """Rest shapes, masses and deformation gradients of a state."""
+
+    def __init__(self, case, seed):
+        sc = _scene(case)
+        x, v, _, frame = _state(case, sc, seed)
+        dev = _device()
+        self.free, self.dt = torch.from_numpy(~sc.dirichlet_mask).to(dev), sc.dt
+        self.x, rest = torch.from_numpy(x).to(dev), torch.from_numpy(sc.x).to(dev)
+        t = self.t = torch.from_numpy(sc.tets.astype(np.int64)).to(dev)
+        self.rest = rest
+        dm = torch.stack([rest[t[:, k]] - rest[t[:, 0]] for k in (1, 2, 3)], 2)
+        ds = torch.stack([self.x[t[:, k]] - self.x[t[:, 0]] for k in (1, 2, 3)], 2)
+        self.vol = (dm[:, :, 0] * torch.linalg.cross(dm[:, :, 1], dm[:, :, 2])).sum(1) / 6
+        # rows of the inverse: cross products of the columns over the determinant
+        self.inv = torch.stack([torch.linalg.cross(dm[:, :, (j + 1) % 3], dm[:, :, (j + 2) % 3]) for j in range(3)],
+                               1) / (6 * self.vol)[:, None, None]
+        self.F = (ds[:, :, :, None] * self.inv[:, None]).sum(2)
+        E, nu = torch.from_numpy(sc.youngs).to(dev), torch.from_numpy(sc.poisson).to(dev)
+        self.la, self.mu = E * nu / ((1 + nu) * (1 - 2 * nu)), E / (2 * (1 + nu))
+        F = self.F
+        self.cof = torch.stack([torch.linalg.cross(F[:, (i + 1) % 3], F[:, (i + 2) % 3]) for i in range(3)], 1)
+        self.J = (F[:, 0] * self.cof[:, 0]).sum(1)
+        self.mass = torch.zeros(len(x), dtype=torch.float64, device=dev)
+        for k in range(4):
+            self.mass.index_add_(0, t[:, k], self.vol * torch.from_numpy(sc.density).to(dev) / 4)
+        # x moved by dt v in the step before, so the next inertial increment
+        # is x - (x - dt v) + dt^2 g; the fixed vertices go to new positions
+        inc = x - (x - sc.dt * v)
+        inc[:, 1] += sc.dt * sc.dt * sc.gravity
+        inc[sc.dirichlet_mask] = sc.dirichlet_rows(frame * sc.dt)[1] - x[sc.dirichlet_mask]
+        self.inc = torch.from_numpy(inc).to(dev)
+
+
 def _exact_linesearch(case, seed):
     """The inertia and the elastic energy at the start of the search."""
-    sc = _scene(case)
-    x, v, _, frame = _state(case, sc, seed)
-    free, dt = ~sc.dirichlet_mask, sc.dt
-    X, R = torch.from_numpy(x), torch.from_numpy(sc.x)
-    t = torch.from_numpy(sc.tets.astype(np.int64))
-    dm = torch.stack([R[t[:, k]] - R[t[:, 0]] for k in (1, 2, 3)], 2)
-    ds = torch.stack([X[t[:, k]] - X[t[:, 0]] for k in (1, 2, 3)], 2)
-    vol = torch.linalg.det(dm) / 6
-    F = ds @ torch.linalg.inv(dm)
-    E, nu = torch.from_numpy(sc.youngs), torch.from_numpy(sc.poisson)
-    la, mu = E * nu / ((1 + nu) * (1 - 2 * nu)), E / (2 * (1 + nu))
-    logj = torch.log(torch.linalg.det(F))
-    psi = mu / 2 * ((F * F).sum((1, 2)) - 3) - mu * logj + la / 2 * logj ** 2
-    # x moved by dt v in the step before, so the next inertial increment is
-    # (x - (x - dt v)) + dt^2 g; the fixed vertices go to their new positions
-    inc = (x - (x - dt * v))
-    inc[:, 1] += dt * dt * sc.gravity
-    inc[~free] = sc.dirichlet_rows(frame * dt)[1] - x[~free]
-    mass = torch.zeros(len(x), dtype=torch.float64)
-    for k in range(4):
-        mass.index_add_(0, t[:, k], vol * torch.from_numpy(sc.density) / 4)
-    inertia = 0.5 * (mass * (torch.from_numpy(inc) ** 2).sum(1)).sum()
+    e = _Elastic(case, seed)
+    logj = torch.log(e.J)
+    psi = e.mu / 2 * ((e.F * e.F).sum((1, 2)) - 3) - e.mu * logj + e.la / 2 * logj ** 2
+    inertia = 0.5 * (e.mass * (e.inc ** 2).sum(1)).sum()
     none = dict.fromkeys(("counts", "hits", "barrier0", "E0", "alpha", "bounds", "parts", "E", "x"))
-    return none | {"inertia0": float(inertia), "elastic0": float((psi * vol).sum() * dt * dt)}
+    return none | {"inertia0": float(inertia), "elastic0": float((psi * e.vol).sum() * e.dt * e.dt)}
+
+
+def _dot(a, b):
+    return (a * b).sum(-1)
+
+
+def _cross(a, b):
+    return torch.linalg.cross(a, b)
+
+
+# squared distances, of points p[..., k, 3]
+def _point_point(p):
+    return _dot(p[..., 0, :] - p[..., 1, :], p[..., 0, :] - p[..., 1, :])
+
+
+def _point_line(p):
+    n, e = _cross(p[..., 1, :] - p[..., 0, :], p[..., 2, :] - p[..., 0, :]), p[..., 2, :] - p[..., 1, :]
+    return _dot(n, n) / _dot(e, e)
+
+
+def _point_plane(p):
+    n = _cross(p[..., 2, :] - p[..., 1, :], p[..., 3, :] - p[..., 1, :])
+    return _dot(p[..., 0, :] - p[..., 1, :], n) ** 2 / _dot(n, n)
+
+
+def _line_line(p):
+    n = _cross(p[..., 1, :] - p[..., 0, :], p[..., 3, :] - p[..., 2, :])
+    return _dot(p[..., 2, :] - p[..., 0, :], n) ** 2 / _dot(n, n)
+
+
+def _near(lo_a, hi_a, lo_b, hi_b, dh):
+    """Index pairs of boxes that overlap within dh."""
+    out, step = [], max(1, 200_000_000 // max(1, len(lo_b)))
+    for i in range(0, len(lo_a), step):
+        ok = torch.ones(len(lo_a[i:i + step]), len(lo_b), dtype=torch.bool, device=lo_a.device)
+        for d in range(3):
+            ok &= lo_a[i:i + step, None, d] < hi_b[None, :, d] + dh
+            ok &= lo_b[None, :, d] - dh < hi_a[i:i + step, None, d]
+        a, b = torch.nonzero(ok, as_tuple=True)
+        out.append(torch.stack([a + i, b]))
+    return torch.cat(out, 1)
+
+
+def _point_triangle_type(p):
+    """0-2 a vertex, 3-5 an edge, 6 the face of the triangle nearest to the point."""
+    P, T = p[:, 0], [p[:, 1], p[:, 2], p[:, 3]]
+    n = _cross(T[1] - T[0], T[2] - T[0])
+    s, side = [], []
+    for k in range(3):
+        e, d = T[(k + 1) % 3] - T[k], P - T[k]
+        s.append(_dot(e, d) / _dot(e, e))
+        side.append(_dot(_cross(e, n), d))
+    kind = torch.full((len(p),), 6, device=p.device)
+    for k in (2, 1, 0):  # vertex k: before edge k's start, past the previous edge's end
+        kind = torch.where((s[k] <= 0) & (s[(k + 2) % 3] >= 1), k, kind)
+    for k in (2, 1, 0):
+        beyond = side[k] > 0 if k == 2 else side[k] >= 0
+        kind = torch.where((s[k] > 0) & (s[k] < 1) & beyond, 3 + k, kind)
+    return kind
+
+
+def _edge_edge_type(p):
+    """3 i + j: the nearest features of two edges, i (j) = 0, 1 the ends, 2 the inside of the first (second)."""
+    u, v, w = p[:, 1] - p[:, 0], p[:, 3] - p[:, 2], p[:, 0] - p[:, 2]
+    a, b, c, d, e = _dot(u, u), _dot(u, v), _dot(v, v), _dot(u, w), _dot(v, w)
+    D = a * c - b * b
+    sN, n = b * e - c * d, _cross(u, v)
+    parallel = (sN > 0) & (sN < D) & (a * e - b * d > 0) & (a * e - b * d < D) & \
+        ((_dot(n, w) == 0) | (_dot(n, n) < 1e-20 * a * c))
+    start, end = (sN <= 0) | (parallel & (sN < D / 2)), (sN >= D) | (parallel & (sN >= D / 2))
+    end &= ~start
+    tN = torch.where(start, e, torch.where(end, e + b, a * e - b * d))
+    tD = torch.where(start | end, c, D)
+    i = torch.where(start, 0, torch.where(end, 1, 2))
+    low, high = tN <= 0, tN >= tD
+    q = torch.where(low, -d, -d + b)
+    i = torch.where(low | high, torch.where(q <= 0, 0, torch.where(q >= a, 1, 2)), i)
+    return 3 * i + torch.where(low, 0, torch.where(high, 1, 2))
+
+
+def _contacts(e, sc):
+    """(distance, vertices of the row, places of the distance's points in it,
+    mollified) for every kind of contact within the barrier distance, rows unique."""
+    x, dh, dev = e.x, sc.dhat, e.x.device
+    points, edges, tris = (torch.from_numpy(a.astype(np.int64)).to(dev) for a in sc.boundary)
+    rows = {}
+
+    def add(name, ids):
+        rows.setdefault(name, []).append(ids)
+
+    lo, hi = x[tris].amin(1), x[tris].amax(1)
+    a, b = _near(x[points], x[points], lo, hi, dh)
+    q = torch.cat([points[a][:, None], tris[b]], 1)
+    q = q[(q[:, 1:] != q[:, :1]).all(1)]
+    kind = _point_triangle_type(x[q])
+    for k in range(7):
+        c = q[kind == k]
+        if k < 3:
+            c, f, name = c[:, [0, 1 + k]], _point_point, "pp"
+        elif k < 6:
+            c, f, name = c[:, [0, 1 + k - 3, 1 + (k - 2) % 3]], _point_line, "pe"
+        else:
+            f, name = _point_plane, "pt"
+        add(name, c[f(x[c]) < dh * dh])
+    lo, hi = x[edges].amin(1), x[edges].amax(1)
+    a, b = _near(lo, hi, lo, hi, dh)
+    q = torch.cat([edges[a], edges[b]], 1)[a < b]
+    q = q[(q[:, :2, None] != q[:, None, 2:]).all(2).all(1)]
+    kind = _edge_edge_type(x[q])
+    n, r = _cross(x[q[:, 1]] - x[q[:, 0]], x[q[:, 3]] - x[q[:, 2]]), e.rest
+    moll = _dot(n, n) < 1e-3 * _point_point(r[q[:, :2]]) * _point_point(r[q[:, 2:]])
+    for k in range(9):
+        i, j = divmod(k, 3)
+        c, m = q[kind == k], moll[kind == k]
+        if i < 2 and j < 2:
+            c, at, f, name = c[:, [i, 1 - i, 2 + j, 3 - j]], [0, 2], _point_point, "pp"
+        elif i < 2:
+            c, at, f, name = c[:, [i, 1 - i, 2, 3]], [0, 2, 3], _point_line, "pe"
+        elif j < 2:
+            c, at, f, name = c[:, [2 + j, 3 - j, 0, 1]], [0, 2, 3], _point_line, "pe"
+        else:
+            at, f, name = [0, 1, 2, 3], _line_line, "ee"
+        near = f(x[c[:, at]]) < dh * dh
+        add(name, c[near & ~m][:, at])
+        add(name + "m", c[near & m])
+    form = {"pp": (_point_point, [0, 1], False), "pe": (_point_line, [0, 1, 2], False),
+            "pt": (_point_plane, [0, 1, 2, 3], False), "ee": (_line_line, [0, 1, 2, 3], False),
+            "ppm": (_point_point, [0, 2], True), "pem": (_point_line, [0, 2, 3], True),
+            "eem": (_line_line, [0, 1, 2, 3], True)}
+    for name, parts in rows.items():
+        ids = torch.cat(parts)
+        if len(ids):
+            f, at, m = form[name]
+            yield f, torch.unique(ids, dim=0), at, m
+
+
+def _kappa(sc, mass):
+    """The barrier's stiffness of a scene, from its mean mass."""
+    h, d = sc.dhat ** 2, 1e-16
+    second = (-2 * math.log(d / h) - 4 * (d - h) / d) + ((d - h) / d) ** 2
+    return 10 * 1e13 * float(mass.mean()) / (4e-16 * second)
+
+
+def _contact_terms(e, sc):
+    """(vertices, gradient, projected Hessian) of every contact row."""
+    h, kappa = sc.dhat ** 2, _kappa(sc, e.mass)
+    for f, ids, at, moll in _contacts(e, sc):
+        k = ids.shape[1]
+
+        def energy(p, eps):
+            p = p.reshape(k, 3)
+            d = f(p[at])
+            b = -kappa * (d - h) ** 2 * torch.log(d / h)
+            if moll:
+                n = _cross(p[1] - p[0], p[3] - p[2])
+                r = _dot(n, n) / eps
+                b = b * (2 - r) * r
+            return b
+
+        p, rest = e.x[ids].reshape(-1, 3 * k), e.rest[ids]
+        eps = 1e-3 * _point_point(rest[:, :2]) * _point_point(rest[:, 2:]) if moll else torch.ones_like(p[:, 0])
+        g = torch.func.vmap(torch.func.grad(energy))(p, eps)
+        H = torch.func.vmap(torch.func.hessian(energy))(p, eps)
+        lam, V = np.linalg.eigh(((H + H.transpose(1, 2)) / 2).cpu().numpy())
+        H = (V * np.maximum(lam, 0)[:, None, :]) @ V.transpose(0, 2, 1)
+        yield ids, g, torch.from_numpy(H).to(p.device)
+
+
+def _elastic_hessians(e):
+    """The projected 12 x 12 Hessians of the tets: the Hessian over the
+    singular values is projected, and each 2 x 2 twist block by its closed
+    form, which for a negative smaller eigenvalue keeps b^2 / (a + |b|)."""
+    lam, V = np.linalg.eigh((e.F.transpose(1, 2)[..., None] * e.F[:, None]).sum(2).cpu().numpy())
+    V = torch.from_numpy(V).to(e.F.device)
+    U = (e.F[:, :, :, None] * V[:, None]).sum(2)
+    s = torch.sqrt((U * U).sum(1))
+    U = U / s[:, None]
+    lp, la, mu = torch.log(e.J), e.la, e.mu
+    M = torch.zeros(len(s), 9, 9, dtype=torch.float64, device=s.device)
+    S = la[:, None, None] / (s[:, :, None] * s[:, None, :])
+    S[:, range(3), range(3)] = mu[:, None] * (1 + s ** -2) - la[:, None] * s ** -2 * (lp[:, None] - 1)
+    minor = S[:, 0, 0] * S[:, 1, 1] - S[:, 0, 1] ** 2
+    det = (S[:, 0] * _cross(S[:, 1], S[:, 2])).sum(1)
+    bad = torch.nonzero((S[:, 0, 0] <= 0) | (minor <= 0) | (det <= 0))[:, 0]
+    if len(bad):
+        w, Q = np.linalg.eigh(S[bad].cpu().numpy())
+        S[bad] = torch.from_numpy((Q * np.maximum(w, 0)[:, None]) @ Q.transpose(0, 2, 1)).to(s.device)
+    for i in range(3):
+        for j in range(3):
+            M[:, 4 * i, 4 * j] = S[:, i, j]
+    g = mu[:, None] * (s - 1 / s) + la[:, None] / s * lp[:, None]
+    for i, j in ((0, 1), (1, 2), (2, 0)):
+        left = (mu + (mu - la * lp) / (s[:, i] * s[:, j])) / 2
+        right = (g[:, i] + g[:, j]) / (2 * (s[:, i] + s[:, j]))
+        a, b = left + right, left - right
+        cut = a - b.abs() < 0
+        c = torch.where(cut, b * b / (a + b.abs()), a)
+        d = torch.where(cut, c * torch.sign(b), b)
+        p, q = 3 * i + j, 3 * j + i
+        M[:, p, p], M[:, q, q], M[:, p, q], M[:, q, p] = c, c, d, d
+    # vertex a's share of w_(k,l) = u_k v_l^T: sum_j B[a][j] V[j][l] times U[:, k]
+    B = torch.cat([-e.inv.sum(1, keepdim=True), e.inv], 1)
+    BV = (B[:, :, :, None] * V[:, None]).sum(2)
+    Z = (U[:, None, :, :, None] * BV[:, :, None, None, :]).reshape(len(s), 12, 9)
+    return (Z @ M) @ Z.transpose(1, 2).contiguous() * (e.dt ** 2 * e.vol)[:, None, None]
+
+
+def _exact_direction(case, seed):
+    """The right-hand side and the solution of the projected Newton system,
+    by conjugate gradients in 64 bits to the end of their accuracy."""
+    e, sc = _Elastic(case, seed), _scene(case)
+    nv, dev = len(e.x), e.x.device
+    P = e.mu[:, None, None] * e.F + ((e.la * torch.log(e.J) - e.mu) / e.J)[:, None, None] * e.cof
+    B = torch.cat([-e.inv.sum(1, keepdim=True), e.inv], 1)
+    g = (P[:, None] * B[:, :, None, :]).sum(3) * (e.dt ** 2 * e.vol)[:, None, None]
+    terms = [(e.t, g.reshape(-1, 12), _elastic_hessians(e))] + list(_contact_terms(e, sc))
+    b = e.mass[:, None] * e.inc
+    D = torch.zeros(nv, 3, 3, dtype=torch.float64, device=dev)
+    D[:, range(3), range(3)] = e.mass[:, None]
+    for ids, gr, H in terms:
+        k = ids.shape[1]
+        b = b.index_add(0, ids.reshape(-1), -gr.reshape(-1, 3))
+        H4 = H.reshape(-1, k, 3, k, 3)
+        for a in range(k):
+            D.index_add_(0, ids[:, a], H4[:, a, :, a])
+    free = e.free[:, None].double()
+    rhs = b * free
+
+    def product(p):
+        q = e.mass[:, None] * p
+        for ids, _, H in terms:
+            q = q.index_add(0, ids.reshape(-1), (H * p[ids].reshape(len(ids), 1, -1)).sum(2).reshape(-1, 3))
+        return q * free
+
+    inv = torch.linalg.inv(D.cpu()).to(dev)
+    fixed = e.inc * (1 - free)
+    r = rhs - product(fixed)
+    x, goal = torch.zeros_like(r), float((r * r).sum()) * 1e-26
+    for _ in range(3):  # restarts with the true residual
+        z = (inv * r[:, None]).sum(2) * free
+        p, rz = z, (r * z).sum()
+        for it in range(4000):
+            q = product(p)
+            alpha = rz / (p * q).sum()
+            x, r = x + alpha * p, r - alpha * q
+            if it % 16 == 15 and float((r * r).sum()) < goal:
+                break
+            z = (inv * r[:, None]).sum(2) * free
+            new = (r * z).sum()
+            p, rz = z + (new / rz) * p, new
+        r = rhs - product(fixed + x)
+    x = x + fixed
+    return {"counts": None, "done": None, "rhs": rhs.cpu(), "direction": x.cpu()}
 
 
 def exact(case, seed):
-    """The network, and the parts of the energy that need no contact search;
-    directions, steps and times of impact depend on the projected Hessians,
-    the solver's tolerance and the conservative bounds."""
-    if case["kind"] == "mlp":
+    """The network, the directions, and the parts of the energy that need no
+    contact search.  A step ends wherever its Newton tolerance lets it, a time
+    of impact is a conservative bound, and the warm start's features are not
+    restated here."""
+    kind = case["kind"]
+    if kind == "mlp":
         return _exact_mlp(case, seed)
-    if case["kind"] == "linesearch":
+    if kind == "linesearch":
         return _exact_linesearch(case, seed)
+    if kind == "direction":
+        return _exact_direction(case, seed)
     return None
