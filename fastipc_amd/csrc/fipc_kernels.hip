@@ -454,41 +454,44 @@ __device__ __forceinline__ void wave_sync()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// contact rows: a group of G lanes per row (G = 8 for PP, 16 otherwise).
-// The projection onto the positive semi-definite cone (makePD semantics,
-// UTILS.h:7-25: V max(L, 0) V^T of the eigen-decomposition) runs a parallel
-// cyclic Jacobi on the matrix padded to M = N rounded up to even (a zero row
-// and column, never rotated): lane l < M owns row l, a round applies the M / 2
-// disjoint rotations of the pairs (i, M-1-i) at once, A <- J^T A J and
-// V <- V J, then relabels the indices by the round-robin rotation rr_next, so
-// every round is the same code with static register indices (the Brent-Luk
-// arrangement); rows move between lanes, and the columns of J are exchanged,
-// through LDS.  A pair rotates when |a_pq| > 1e-17 |A|_F; sweeps (M - 1
-// rounds) stop once a whole sweep rotates no pair, after at most max_sweeps.
-// LDS of one contact-assembly block: per lane group the M x M matrix and the
-// two coefficient columns, sized for the largest row (M = 12, G = 16)
-#define CONTACT_LDS ((TPB / 16) * (144 + 2 * 12))
+// Contact rows in two launches over all seven types (so that the types, each
+// latency-bound, overlap instead of queueing), a group of G lanes per row
+// (G = 8 for PP, 16 otherwise):
+//  - k_contact_gh evaluates the row's gradient and Hessian; lane l < N stores
+//    row l of the Hessian and entry l of the gradient;
+//  - k_contact projects the Hessian in place.
+// The evaluation holds a whole Hessian in registers (one wave per SIMD).  In
+// one launch with it the projection, the longer part, ran one wave per SIMD
+// too, and 5,000 rows took two rounds of the chip.  29,367 rows (27 stacked
+// cubes of 16^3): 739 us in one launch, 53 + 373 us in two; 4,175 rows (the
+// 1M-tet slab): 160 against 17 + 111 us; 520 rows: 80 us both ways (one round:
+// the latency of about 100 dependent rotation rounds).
+struct ContactBatch {
+    const int* rows[NTYPES];
+    double* H[NTYPES];
+    float* Hf[NTYPES];            // null unless FP32 copies are wanted
+    unsigned char* c64[NTYPES];
+    double* cgrad[NTYPES];        // row gradients, N per row
+    int n[NTYPES];
+    int goff[NTYPES + 1];         // block ranges of the types in k_contact_gh
+    int boff[NTYPES + 1];         // and in k_contact
+};
+constexpr int GH_TPB = 64;  // one wave per block
 template <int KIND>
-__device__ __forceinline__ void contact_row(int n, const int* __restrict__ rows, const double* __restrict__ x,
-                                            const double* __restrict__ x0, double dHat2, double kappa,
-                                            double* __restrict__ Hout, double* cgrad, double* Eout,
-                                            double* gout, int project, int accumulate, int max_sweeps, int gid,
-                                            double* lds, float* __restrict__ Hf, unsigned char* __restrict__ c64)
+__device__ __forceinline__ void contact_gh(int n, int gid, const int* __restrict__ rows, const double* __restrict__ x,
+                                           const double* __restrict__ x0, double dHat2, double kappa,
+                                           double* __restrict__ Hout, double* __restrict__ cgrad, double* Eout,
+                                           unsigned char* __restrict__ c64)
 {
     using KI = KindInfo<KIND>;
     constexpr int N = KI::N, G = KI::G;
-    constexpr int M = (N + 1) & ~1;
-    int r = gid / G, l = gid % G, grp = (int)threadIdx.x / G;
-    if (r >= n) return;  // uniform over the lanes of a row
-    const bool act = l < N;
-    double* A = lds + grp * (M * M + 2 * M);
-    double* jd = A + M * M;
-    double* jo = jd + M;
+    const int r = gid / G, l = gid % G;
+    if (r >= n) return;
     int id[4];
     v3 px[4], p0[4];
     load_row<KIND>(rows, r, x, x0, id, px, p0);
     double g[N], H[N * N];
-    double E = constraint_gH<KIND>(px, p0, dHat2, kappa, g, H);
+    const double E = constraint_gH<KIND>(px, p0, dHat2, kappa, g, H);
     // own row, from the upper triangle
     double o[N];
 #pragma unroll
@@ -499,171 +502,35 @@ __device__ __forceinline__ void contact_row(int n, const int* __restrict__ rows,
 #pragma unroll
             for (int k = 0; k < N; k++) o[k] = k >= L ? H[L * N + k] : H[k * N + L];
         }
-    double out[N];
-    if (project) {
-        // derivative-only arithmetic: contraction into FMA is allowed here
-#pragma clang fp contract(fast)
-        const bool pos = l < M;
-        double a[M], v[M];
-#pragma unroll
-        for (int k = 0; k < M; k++) {
-            a[k] = k < N ? o[k] : 0.0;
-            v[k] = k == l ? 1.0 : 0.0;
-        }
-        double f = 0.0;
-#pragma unroll
-        for (int k = 0; k < M; k++) f += a[k] * a[k];
-#pragma unroll
-        for (int mm = G / 2; mm > 0; mm >>= 1) f += __shfl_xor(f, mm, G);
-        const double tiny = 1e-17 * sqrt(f);
-        if (pos) {
-#pragma unroll
-            for (int k = 0; k < M; k++) A[l * M + k] = a[k];
-        }
-        wave_sync();
-        const unsigned long long gmask = ((1ull << G) - 1) << (((int)threadIdx.x % 64) / G * G);
-        const int m = M - 1 - l;
-        const int dest = l == 0 ? 0 : (l == M - 1 ? 1 : l + 1);
-        for (int sweep = 0; sweep < max_sweeps; sweep++) {
-            bool rot = false;
-#pragma unroll 1
-            for (int rd = 0; rd < M - 1; rd++) {
-                double c = 1.0, s = 0.0, t = 0.0, app = 0.0, aqq = 0.0, apq = 0.0;
-                double w[M];
-#pragma unroll
-                for (int k = 0; k < M; k++) w[k] = 0.0;
-                if (pos) {
-                    int p = min(l, m), q = max(l, m);
-                    app = A[p * M + p];
-                    aqq = A[q * M + q];
-                    apq = A[p * M + q];
-#pragma unroll
-                    for (int k = 0; k < M; k++) w[k] = A[m * M + k];
-                }
-                const bool did = pos && fabs(apq) > tiny;
-                if (did) {
-                    double theta = (aqq - app) / (2.0 * apq);
-                    t = fabs(theta) > 1e150 ? 0.5 / theta
-                      : (theta >= 0 ? 1.0 : -1.0) / (fabs(theta) + sqrt(theta * theta + 1.0));
-                    c = 1.0 / sqrt(t * t + 1.0);
-                    s = t * c;
-                }
-                // column l of J: J[l][l] = c, J[m][l] = -s (l < m) or s (l > m)
-                const double cl = c, sl = l < m ? -s : s;
-                if (pos) { jd[l] = cl; jo[l] = sl; }
-                wave_sync();
-                double u[M];
-#pragma unroll
-                for (int k = 0; k < M; k++) u[k] = cl * a[k] + sl * w[k];
-                double an[M], vn[M];
-#pragma unroll
-                for (int k = 0; k < M; k++) {
-                    double ck = jd[k], sk = jo[k];
-                    an[k] = ck * u[k] + sk * u[M - 1 - k];
-                    vn[k] = ck * v[k] + sk * v[M - 1 - k];
-                }
-                if (did) {
-                    // the rotated pair's entries, exactly
-                    double dnew = l < m ? app - t * apq : aqq + t * apq;
-#pragma unroll
-                    for (int k = 0; k < M; k++) {
-                        if (k == m) an[k] = 0.0;
-                        if (k == l) an[k] = dnew;
-                    }
-                }
-                rot = rot || did;
-                // relabel the columns (static) and move the row to its new position
-#pragma unroll
-                for (int k = 0; k < M; k++) {
-                    a[rr_next<M>(k)] = an[k];
-                    v[rr_next<M>(k)] = vn[k];
-                }
-                if (pos) {
-#pragma unroll
-                    for (int k = 0; k < M; k++) A[dest * M + k] = a[k];
-                }
-                wave_sync();
-                if (pos) {
-#pragma unroll
-                    for (int k = 0; k < M; k++) a[k] = A[l * M + k];
-                }
-            }
-            if ((__ballot(rot) & gmask) == 0) break;
-        }
-        // eigenvalues clamped at zero; rows of V replace A in LDS
-        double lam = pos ? fmax(A[l * M + l], 0.0) : 0.0;
-        wave_sync();
-        if (pos) {
-#pragma unroll
-            for (int k = 0; k < M; k++) A[l * M + k] = v[k];
-            jd[l] = lam;
-        }
-        wave_sync();
-        double lv[M];
-#pragma unroll
-        for (int k = 0; k < M; k++) lv[k] = v[k] * jd[k];
-#pragma unroll
-        for (int cc = 0; cc < N; cc++) {
-            double sum = 0.0;
-#pragma unroll
-            for (int k = 0; k < M; k++) sum += lv[k] * A[cc * M + k];
-            out[cc] = sum;
-        }
-    } else {
-#pragma unroll
-        for (int k = 0; k < N; k++) out[k] = o[k];
-    }
-    if (!act) return;
+    if (l >= N) return;
     double* Hr = Hout + (size_t)r * N * N + (size_t)l * N;
 #pragma unroll
-    for (int k = 0; k < N; k++) Hr[k] = out[k];
-    if (Hf) {
-        // FP32 copy for the FP32 iterations; rows closer than 1e-2 dHat
-        // (squared distance below 1e-4 dHat^2) are flagged to stay FP64
-        float* Hfr = Hf + (size_t)r * N * N + (size_t)l * N;
-#pragma unroll
-        for (int k = 0; k < N; k++) Hfr[k] = (float)out[k];
-        if (l == 0) c64[r] = constraint_dist(KIND, px) < 1e-4 * dHat2 ? 1 : 0;
-    }
+    for (int k = 0; k < N; k++) Hr[k] = o[k];
+    // the row's gradient at its vertex l / 3 (slot K r + l / 3 of the type),
+    // summed per vertex by k_cv_gather (load_hessian_and_gradient,
+    // NEWTON_IPC.py:546-555)
     double gl = g[0];
 #pragma unroll
     for (int k = 1; k < N; k++)
         if (k == l) gl = g[k];
-    if (accumulate) {
-        // the row's gradient at its vertex l / 3 (slot K r + l / 3 of the
-        // type), summed per vertex by k_cv_gather (load_hessian_and_gradient,
-        // NEWTON_IPC.py:546-555)
-        cgrad[3 * (size_t)r * KI::K + l] = gl;
-    } else {
-        if (l == 0 && Eout) Eout[r] = E;
-        if (gout) gout[(size_t)r * N + l] = gl;
+    cgrad[(size_t)r * N + l] = gl;
+    if (l == 0) {
+        if (Eout) Eout[r] = E;
+        // rows closer than 1e-2 dHat (squared distance below 1e-4 dHat^2)
+        // stay FP64 in the FP32 iterations
+        if (c64) c64[r] = constraint_dist(KIND, px) < 1e-4 * dHat2 ? 1 : 0;
     }
 }
-
-// every constraint type in one launch: blocks [boff[t], boff[t + 1]) run the
-// rows of type t, so the (latency-bound) types overlap instead of queueing
-struct ContactBatch {
-    const int* rows[NTYPES];
-    double* H[NTYPES];
-    float* Hf[NTYPES];            // null unless FP32 copies are wanted
-    unsigned char* c64[NTYPES];
-    double* cgrad[NTYPES];        // slot gradients of the type (accumulate mode)
-    int n[NTYPES];
-    int boff[NTYPES + 1];
-};
-__global__ void __launch_bounds__(TPB) k_contact(ContactBatch cb, const double* __restrict__ x,
-                                                 const double* __restrict__ x0, double dHat2, double kappa,
-                                                 double* Eout, double* gout, int project, int accumulate,
-                                                 int max_sweeps)
+__global__ void __launch_bounds__(GH_TPB) k_contact_gh(ContactBatch cb, const double* __restrict__ x,
+                                                       const double* __restrict__ x0, double dHat2, double kappa,
+                                                       double* Eout)
 {
-    __shared__ double lds[CONTACT_LDS];
     int b = (int)blockIdx.x, t = 0;
-    while (t < NTYPES - 1 && b >= cb.boff[t + 1]) t++;
-    int gid = (b - cb.boff[t]) * TPB + (int)threadIdx.x;
-#define CONTACT_CASE(K)                                                                                            \
-    case K:                                                                                                         \
-        contact_row<K>(cb.n[K], cb.rows[K], x, x0, dHat2, kappa, cb.H[K], cb.cgrad[K], Eout, gout, project,     \
-                       accumulate, max_sweeps, gid, lds, cb.Hf[K], cb.c64[K]);                                      \
+    while (t < NTYPES - 1 && b >= cb.goff[t + 1]) t++;
+    const int gid = (b - cb.goff[t]) * GH_TPB + (int)threadIdx.x;
+#define CONTACT_CASE(K)                                                                                        \
+    case K:                                                                                                    \
+        contact_gh<K>(cb.n[K], gid, cb.rows[K], x, x0, dHat2, kappa, cb.H[K], cb.cgrad[K], Eout, cb.c64[K]); \
         break;
     switch (t) {
         CONTACT_CASE(0)
@@ -676,17 +543,213 @@ __global__ void __launch_bounds__(TPB) k_contact(ContactBatch cb, const double* 
     }
 #undef CONTACT_CASE
 }
-// block ranges of the types with rows (G lanes per row)
-static int contact_blocks(ContactBatch& cb)
+
+// The projection onto the positive semi-definite cone (makePD semantics,
+// UTILS.h:7-25: V max(L, 0) V^T of the eigen-decomposition) runs a parallel
+// cyclic Jacobi on the matrix padded to M = N rounded up to even (a zero row
+// and column, never rotated): lane l < M owns row l, a round applies the M / 2
+// disjoint rotations of the pairs (i, M-1-i) at once, A <- J^T A J and
+// V <- V J, then relabels the indices by the round-robin rotation rr_next, so
+// every round is the same code with static register indices (the Brent-Luk
+// arrangement).  A lane keeps its row, whose index moves instead; the partner's
+// row and the pairs' (c, s) are read through LDS (moving the rows as well and
+// reading both lanes' coefficients, 520 instead of 312 bytes per lane and round,
+// took 438 instead of 373 us for the 29,367 rows; 2 waves per SIMD 428 us, 4 no
+// less than 3).  A pair rotates when |a_pq| > 1e-17 |A|_F; sweeps (M - 1
+// rounds) stop once a whole sweep rotates no pair, after at most max_sweeps.
+// The rotations' products are written as fused multiply-adds, so that the bits
+// do not depend on which products the compiler fuses.
+// LDS of one block: per lane group the matrix and the two coefficient columns,
+// sized for the largest row (M = 12, G = 16); rows of 12 are 14 apart, so that
+// the 16-byte reads of 12 rows fall on different banks.
+__host__ __device__ constexpr int contact_stride(int M) { return M == 12 ? 14 : M; }
+#define CONTACT_LDS ((TPB / 16) * (12 * contact_stride(12) + 2 * 12))
+template <int KIND>
+__device__ __forceinline__ void contact_row(int n, double* __restrict__ H, int max_sweeps, int gid, double* lds,
+                                            float* __restrict__ Hf)
 {
-    int nb = 0;
-    for (int t = 0; t < NTYPES; t++) {
-        int G = kind_dofs(t) <= 8 ? 8 : 16;
-        cb.boff[t] = nb;
-        nb += cb.n[t] ? nblk((long)cb.n[t] * G) : 0;
+    using KI = KindInfo<KIND>;
+    constexpr int N = KI::N, G = KI::G;
+    constexpr int M = (N + 1) & ~1, S = contact_stride(M);
+    int r = gid / G, l = gid % G, grp = (int)threadIdx.x / G;
+    if (r >= n) return;  // uniform over the lanes of a row
+    const bool act = l < N;
+    double* A = lds + grp * (M * S + 2 * M);
+    double* jd = A + M * S;
+    double* jo = jd + M;
+    double* Hr = H + (size_t)r * N * N + (size_t)l * N;
+    double o[N], out[N];
+#pragma unroll
+    for (int k = 0; k < N; k++) o[k] = act ? Hr[k] : 0.0;
+    {
+        // derivative-only arithmetic: contraction into FMA is allowed here
+#pragma clang fp contract(fast)
+        const bool pos = l < M;
+        double a[M], v[M];
+#pragma unroll
+        for (int k = 0; k < M; k++) {
+            a[k] = k < N ? o[k] : 0.0;
+            v[k] = k == l ? 1.0 : 0.0;
+        }
+        double f = 0.0;
+#pragma unroll
+        for (int k = 0; k < M; k++) f = k ? fma(a[k], a[k], f) : a[k] * a[k];
+#pragma unroll
+        for (int mm = G / 2; mm > 0; mm >>= 1) f += __shfl_xor(f, mm, G);
+        const double tiny = 1e-17 * sqrt(f);
+        if (pos) {
+#pragma unroll
+            for (int k = 0; k < M; k++) A[l * S + k] = a[k];
+        }
+        wave_sync();
+        const unsigned long long gmask = ((1ull << G) - 1) << (((int)threadIdx.x % 64) / G * G);
+        for (int sweep = 0; sweep < max_sweeps; sweep++) {
+            bool rot = false;
+            int lab = l;  // the index this lane's row has in the current round
+#pragma unroll 1
+            for (int rd = 0; rd < M - 1; rd++) {
+                // partner index, and the lane that holds its row
+                const int m = M - 1 - lab;
+                int pl = m == 0 ? 0 : m - rd;
+                if (m != 0 && pl < 1) pl += M - 1;
+                double c = 1.0, s = 0.0, t = 0.0, app = 0.0, aqq = 0.0, apq = 0.0;
+                double w[M];
+#pragma unroll
+                for (int k = 0; k < M; k++) w[k] = 0.0;
+                if (pos) {
+                    const bool low = lab < m;
+                    const int p = low ? lab : m, q = low ? m : lab;
+                    const double* Ap = A + (low ? l : pl) * S;
+                    app = Ap[p];
+                    apq = Ap[q];
+                    aqq = A[(low ? pl : l) * S + q];
+#pragma unroll
+                    for (int k = 0; k < M; k++) w[k] = A[pl * S + k];
+                }
+                const bool did = pos && fabs(apq) > tiny;
+                if (did) {
+                    double theta = (aqq - app) / (2.0 * apq);
+                    t = fabs(theta) > 1e150 ? 0.5 / theta
+                      : (theta >= 0 ? 1.0 : -1.0) / (fabs(theta) + sqrt(fma(theta, theta, 1.0)));
+                    c = 1.0 / sqrt(fma(t, t, 1.0));
+                    s = t * c;
+                }
+                // column lab of J: J[lab][lab] = c, J[m][lab] = -s (lab < m)
+                // or s; both lanes of a pair hold the same c and s, so the
+                // lower one's stand for both
+                const double cl = c, sl = lab < m ? -s : s;
+                if (pos && lab < m) { jd[lab] = cl; jo[lab] = sl; }
+                wave_sync();
+                double u[M];
+#pragma unroll
+                for (int k = 0; k < M; k++) u[k] = fma(cl, a[k], sl * w[k]);
+                double an[M], vn[M];
+#pragma unroll
+                for (int k = 0; k < M / 2; k++) {
+                    const int h = M - 1 - k;
+                    const double ck = jd[k], sk = jo[k];
+                    an[k] = fma(ck, u[k], sk * u[h]);
+                    an[h] = fma(ck, u[h], -sk * u[k]);
+                    vn[k] = fma(ck, v[k], sk * v[h]);
+                    vn[h] = fma(ck, v[h], -sk * v[k]);
+                }
+                if (did) {
+                    // the rotated pair's entries, exactly
+                    double dnew = lab < m ? fma(-t, apq, app) : fma(t, apq, aqq);
+#pragma unroll
+                    for (int k = 0; k < M; k++) {
+                        if (k == m) an[k] = 0.0;
+                        if (k == lab) an[k] = dnew;
+                    }
+                }
+                rot = rot || did;
+                // relabel the columns (static) and this lane's row
+#pragma unroll
+                for (int k = 0; k < M; k++) {
+                    a[rr_next<M>(k)] = an[k];
+                    v[rr_next<M>(k)] = vn[k];
+                }
+                lab = lab == 0 ? 0 : (lab == M - 1 ? 1 : lab + 1);
+                if (pos) {
+#pragma unroll
+                    for (int k = 0; k < M; k++) A[l * S + k] = a[k];
+                }
+                wave_sync();
+            }
+            if ((__ballot(rot) & gmask) == 0) break;
+        }
+        // eigenvalues clamped at zero; rows of V replace A in LDS
+        double lam = pos ? fmax(A[l * S + l], 0.0) : 0.0;
+        wave_sync();
+        if (pos) {
+#pragma unroll
+            for (int k = 0; k < M; k++) A[l * S + k] = v[k];
+            jd[l] = lam;
+        }
+        wave_sync();
+        double lv[M];
+#pragma unroll
+        for (int k = 0; k < M; k++) lv[k] = v[k] * jd[k];
+#pragma unroll
+        for (int cc = 0; cc < N; cc++) {
+            double sum = 0.0;
+#pragma unroll
+            for (int k = 0; k < M; k++) sum += lv[k] * A[cc * S + k];
+            out[cc] = sum;
+        }
     }
+    if (!act) return;
+#pragma unroll
+    for (int k = 0; k < N; k++) Hr[k] = out[k];
+    if (Hf) {  // FP32 copy for the FP32 iterations
+        float* Hfr = Hf + (size_t)r * N * N + (size_t)l * N;
+#pragma unroll
+        for (int k = 0; k < N; k++) Hfr[k] = (float)out[k];
+    }
+}
+
+// blocks [boff[t], boff[t + 1]) run the rows of type t
+__global__ void __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(3)))
+k_contact(ContactBatch cb, int max_sweeps)
+{
+    __shared__ double lds[CONTACT_LDS];
+    int b = (int)blockIdx.x, t = 0;
+    while (t < NTYPES - 1 && b >= cb.boff[t + 1]) t++;
+    int gid = (b - cb.boff[t]) * TPB + (int)threadIdx.x;
+#define CONTACT_CASE(K)                                                     \
+    case K:                                                                 \
+        contact_row<K>(cb.n[K], cb.H[K], max_sweeps, gid, lds, cb.Hf[K]); \
+        break;
+    switch (t) {
+        CONTACT_CASE(0)
+        CONTACT_CASE(1)
+        CONTACT_CASE(2)
+        CONTACT_CASE(3)
+        CONTACT_CASE(4)
+        CONTACT_CASE(5)
+        CONTACT_CASE(6)
+    }
+#undef CONTACT_CASE
+}
+// both launches on st; the second only with project
+static int contact_launch(ContactBatch& cb, const double* x, const double* x0, double dHat2, double kappa,
+                          double* Eout, int project, hipStream_t st)
+{
+    int ng = 0, nb = 0;
+    for (int t = 0; t < NTYPES; t++) {
+        const long lanes = (long)cb.n[t] * (kind_dofs(t) <= 8 ? 8 : 16);
+        cb.goff[t] = ng;
+        cb.boff[t] = nb;
+        ng += nblk(lanes, GH_TPB);
+        nb += nblk(lanes);
+    }
+    cb.goff[NTYPES] = ng;
     cb.boff[NTYPES] = nb;
-    return nb;
+    if (!nb) return FIPC_OK;
+    k_contact_gh<<<ng, GH_TPB, 0, st>>>(cb, x, x0, dHat2, kappa, Eout);
+    if (project) k_contact<<<nb, TPB, 0, st>>>(cb, 20);
+    HIPCHK(hipGetLastError());
+    return FIPC_OK;
 }
 
 // ---- contact vertices: the slots of every row keyed by vertex ----
@@ -1934,7 +1997,7 @@ static int build_contact_vertices(fipc_ctx* c, hipStream_t st)
     HIPCHK(hipGetLastError());
     return FIPC_OK;
 }
-static int launch_contacts(fipc_ctx* c, int accumulate, hipStream_t st)
+static int launch_contacts(fipc_ctx* c, hipStream_t st)
 {
     if (c->cv_version != c->cons_version) STCHK(build_contact_vertices(c, st));
     ContactBatch cb;
@@ -1951,11 +2014,9 @@ static int launch_contacts(fipc_ctx* c, int accumulate, hipStream_t st)
         cb.c64[t] = c->precision == 1 ? c->c64[t].p : nullptr;
         cb.cgrad[t] = c->cgrad.p + 3 * (size_t)c->soff[t];
     }
-    int nb = contact_blocks(cb);
-    if (!nb) return FIPC_OK;
-    k_contact<<<nb, TPB, 0, st>>>(cb, c->x.p, c->x0.p, c->dHat2, c->kappa, nullptr, nullptr, 1, accumulate, 20);
-    HIPCHK(hipGetLastError());
     const int S = c->soff[NTYPES];
+    if (!S) return FIPC_OK;
+    STCHK(contact_launch(cb, c->x.p, c->x0.p, c->dHat2, c->kappa, nullptr, 1, st));
     k_cv_gather<<<nblk((long)CV_G * S), TPB, 0, st>>>(c->cv_count.p, c->cv_vert.p, c->cv_ptr.p, c->cv_slot.p,
                                               contact_slots(c, false), c->cgrad.p, c->rhs.p, c->cdiag.p);
     HIPCHK(hipGetLastError());
@@ -1986,7 +2047,7 @@ extern "C" int fipc_assemble(fipc_ctx* c, int precision)
     HIPCHK(hipEventRecord(c->ev_rhs, c->s));
     HIPCHK(hipStreamWaitEvent(c->s2, c->ev_rhs, 0));
     STCHK(fipc_tm_begin(c, TM_CONTACT, c->s2));
-    STCHK(launch_contacts(c, 1, c->s2));
+    STCHK(launch_contacts(c, c->s2));
     STCHK(fipc_tm_end(c, TM_CONTACT, c->s2));
     HIPCHK(hipEventRecord(c->ev_contact, c->s2));
     // FP64: per-tet FP64 records, each block sums its tets in index order.
@@ -2632,11 +2693,9 @@ extern "C" int fipc_batch_constraint(int type, int n, const double* x, const dou
     ContactBatch cb;
     for (int t = 0; t < NTYPES; t++) {
         cb.rows[t] = drows; cb.H[t] = dH; cb.n[t] = t == type ? n : 0;
-        cb.Hf[t] = nullptr; cb.c64[t] = nullptr; cb.cgrad[t] = nullptr;
+        cb.Hf[t] = nullptr; cb.c64[t] = nullptr; cb.cgrad[t] = dg;
     }
-    int nb = contact_blocks(cb);
-    k_contact<<<nb, TPB>>>(cb, dx, dx0, dHat2, kappa, dE, dg, project, 0, 20);
-    HIPCHK(hipGetLastError());
+    STCHK(contact_launch(cb, dx, dx0, dHat2, kappa, dE, project, nullptr));
     HIPCHK(hipDeviceSynchronize());
     if (E) HIPCHK(hipMemcpy(E, dE, (size_t)n * 8, hipMemcpyDeviceToHost));
     if (g) HIPCHK(hipMemcpy(g, dg, (size_t)n * N * 8, hipMemcpyDeviceToHost));
