@@ -141,12 +141,7 @@ struct fipc_ctx {
     int raw_count[NTYPES] = {0};
     DVec<int> rows[NTYPES];
     DVec<int> rows_tmp;    // the sort of the four-index types writes here, then swaps
-    DVec<double> cH[NTYPES];
-    // FP32 Hessian: FP32 copies of the contact rows' projected Hessians for
-    // the FP32 iterations, and per row a flag (1) for the rows closer than
-    // 1e-2 dHat, whose FP64 Hessian those iterations keep using
-    DVec<float> cHf[NTYPES];
-    DVec<unsigned char> c64[NTYPES];
+    DVec<double> cH[NTYPES];  // the rows' unprojected Hessians, between the assembly's two contact launches
     // Contact vertices: every (row, vertex) slot of the seven types, slot
     // s = soff[t] + K_t r + a, keyed by its vertex and stably sorted, so the
     // slots of a vertex are contiguous and in (type, row, vertex) order;
@@ -158,7 +153,14 @@ struct fipc_ctx {
     // when the rows changed (cv_version = cons_version of the build).
     int soff[NTYPES + 1] = {0};
     DVec<int> cv_keys, cv_vals, cv_keys2, cv_slot, cv_head, cv_vert, cv_ptr, cv_count;
-    DVec<double> cgrad;    // per slot the row's gradient at that vertex (3)
+    // per slot, at its place in that order (cv_place[s]): the row's points, its
+    // Hessian rows at the vertex (36 values; in FP32 mode also an FP32 copy for
+    // the FP32 iterations, which keep the FP64 values of the rows closer than
+    // 1e-2 dHat) and the row's gradient there (3)
+    DVec<int> cv_place, cv_meta;
+    DVec<int4> cv_ids;
+    DVec<double> cv_H, cgrad;
+    DVec<float> cv_Hf;
     unsigned long long cv_version = 0;
     DVec<unsigned long long> keys_pp, keys_pe, keys_tmp;
     DVec<int> counters;    // NTYPES raw append counters + misc

@@ -454,6 +454,21 @@ __device__ __forceinline__ void wave_sync()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// What the products read of a contact slot (a (row, vertex) pair; see
+// fipc_ctx), at the slot's place in the order sorted by vertex, so that the
+// lanes of a contact vertex find it in a few contiguous loads: the row's
+// points, for each point the 3x3 block of the row's projected Hessian that
+// couples it to the vertex (row-major, 9 per point; an FP32 copy for the FP32
+// iterations), and the vertex's gradient.
+struct SlotData {
+    int4* ids;      // the row's points, -1 past the last
+    int* meta;      // K | the vertex's place in the row << 4 | SLOT_KEEP64
+    double* H;      // 4 x 9 per slot
+    float* Hf;      // the same, or null
+    double* g;      // 3 per slot
+};
+constexpr int SLOT_KEEP64 = 256;  // the row keeps its FP64 Hessian in the FP32 iterations
+
 // Contact rows in two launches over all seven types (so that the types, each
 // latency-bound, overlap instead of queueing), a group of G lanes per row
 // (G = 8 for PP, 16 otherwise):
@@ -468,25 +483,28 @@ __device__ __forceinline__ void wave_sync()
 // the latency of about 100 dependent rotation rounds).
 struct ContactBatch {
     const int* rows[NTYPES];
-    double* H[NTYPES];
-    float* Hf[NTYPES];            // null unless FP32 copies are wanted
-    unsigned char* c64[NTYPES];
-    double* cgrad[NTYPES];        // row gradients, N per row
+    double* H[NTYPES];            // N x N per row: unprojected, then (without slots) projected
     int n[NTYPES];
+    // With pos set (the assembly) the results go to the slots in their sorted
+    // order (see SlotData): slot soff[t] + K r + a of the (row, vertex) pair
+    // to place pos[slot].  Without it g is N per row and H is projected in place.
+    const int* pos;
+    int soff[NTYPES];
+    double* g;
+    SlotData sd;
     int goff[NTYPES + 1];         // block ranges of the types in k_contact_gh
     int boff[NTYPES + 1];         // and in k_contact
 };
 constexpr int GH_TPB = 64;  // one wave per block
 template <int KIND>
-__device__ __forceinline__ void contact_gh(int n, int gid, const int* __restrict__ rows, const double* __restrict__ x,
-                                           const double* __restrict__ x0, double dHat2, double kappa,
-                                           double* __restrict__ Hout, double* __restrict__ cgrad, double* Eout,
-                                           unsigned char* __restrict__ c64)
+__device__ __forceinline__ void contact_gh(const ContactBatch& cb, int gid, const double* __restrict__ x,
+                                           const double* __restrict__ x0, double dHat2, double kappa, double* Eout)
 {
     using KI = KindInfo<KIND>;
-    constexpr int N = KI::N, G = KI::G;
+    constexpr int K = KI::K, N = KI::N, G = KI::G;
+    const int* __restrict__ rows = cb.rows[KIND];
     const int r = gid / G, l = gid % G;
-    if (r >= n) return;
+    if (r >= cb.n[KIND]) return;
     int id[4];
     v3 px[4], p0[4];
     load_row<KIND>(rows, r, x, x0, id, px, p0);
@@ -503,22 +521,29 @@ __device__ __forceinline__ void contact_gh(int n, int gid, const int* __restrict
             for (int k = 0; k < N; k++) o[k] = k >= L ? H[L * N + k] : H[k * N + L];
         }
     if (l >= N) return;
-    double* Hr = Hout + (size_t)r * N * N + (size_t)l * N;
+    double* Hr = cb.H[KIND] + (size_t)r * N * N + (size_t)l * N;
 #pragma unroll
     for (int k = 0; k < N; k++) Hr[k] = o[k];
-    // the row's gradient at its vertex l / 3 (slot K r + l / 3 of the type),
-    // summed per vertex by k_cv_gather (load_hessian_and_gradient,
-    // NEWTON_IPC.py:546-555)
+    // the row's gradient at its vertex l / 3, summed per vertex by
+    // k_cv_gather (load_hessian_and_gradient, NEWTON_IPC.py:546-555)
     double gl = g[0];
 #pragma unroll
     for (int k = 1; k < N; k++)
         if (k == l) gl = g[k];
-    cgrad[(size_t)r * N + l] = gl;
-    if (l == 0) {
-        if (Eout) Eout[r] = E;
+    if (l == 0 && Eout) Eout[r] = E;
+    if (!cb.pos) {
+        cb.g[(size_t)r * N + l] = gl;
+        return;
+    }
+    const int a = l / 3, i = l - 3 * a;
+    const int e = cb.pos[cb.soff[KIND] + K * r + a];
+    cb.sd.g[3 * (size_t)e + i] = gl;
+    if (i == 0) {
         // rows closer than 1e-2 dHat (squared distance below 1e-4 dHat^2)
         // stay FP64 in the FP32 iterations
-        if (c64) c64[r] = constraint_dist(KIND, px) < 1e-4 * dHat2 ? 1 : 0;
+        const int keep = constraint_dist(KIND, px) < 1e-4 * dHat2 ? SLOT_KEEP64 : 0;
+        cb.sd.ids[e] = make_int4(id[0], id[1], K > 2 ? id[2] : -1, K > 3 ? id[3] : -1);
+        cb.sd.meta[e] = K | a << 4 | keep;
     }
 }
 __global__ void __launch_bounds__(GH_TPB) k_contact_gh(ContactBatch cb, const double* __restrict__ x,
@@ -528,9 +553,9 @@ __global__ void __launch_bounds__(GH_TPB) k_contact_gh(ContactBatch cb, const do
     int b = (int)blockIdx.x, t = 0;
     while (t < NTYPES - 1 && b >= cb.goff[t + 1]) t++;
     const int gid = (b - cb.goff[t]) * GH_TPB + (int)threadIdx.x;
-#define CONTACT_CASE(K)                                                                                        \
-    case K:                                                                                                    \
-        contact_gh<K>(cb.n[K], gid, cb.rows[K], x, x0, dHat2, kappa, cb.H[K], cb.cgrad[K], Eout, cb.c64[K]); \
+#define CONTACT_CASE(K)                                \
+    case K:                                            \
+        contact_gh<K>(cb, gid, x, x0, dHat2, kappa, Eout); \
         break;
     switch (t) {
         CONTACT_CASE(0)
@@ -554,8 +579,7 @@ __global__ void __launch_bounds__(GH_TPB) k_contact_gh(ContactBatch cb, const do
 // arrangement).  A lane keeps its row, whose index moves instead; the partner's
 // row and the pairs' (c, s) are read through LDS (moving the rows as well and
 // reading both lanes' coefficients, 520 instead of 312 bytes per lane and round,
-// took 438 instead of 373 us for the 29,367 rows; 2 waves per SIMD 428 us, 4 no
-// less than 3).  A pair rotates when |a_pq| > 1e-17 |A|_F; sweeps (M - 1
+// took 438 instead of 373 us for the 29,367 rows; 2 waves per SIMD 428 us).  A pair rotates when |a_pq| > 1e-17 |A|_F; sweeps (M - 1
 // rounds) stop once a whole sweep rotates no pair, after at most max_sweeps.
 // The rotations' products are written as fused multiply-adds, so that the bits
 // do not depend on which products the compiler fuses.
@@ -565,8 +589,9 @@ __global__ void __launch_bounds__(GH_TPB) k_contact_gh(ContactBatch cb, const do
 __host__ __device__ constexpr int contact_stride(int M) { return M == 12 ? 14 : M; }
 #define CONTACT_LDS ((TPB / 16) * (12 * contact_stride(12) + 2 * 12))
 template <int KIND>
-__device__ __forceinline__ void contact_row(int n, double* __restrict__ H, int max_sweeps, int gid, double* lds,
-                                            float* __restrict__ Hf)
+__device__ __forceinline__ void contact_row(int n, double* __restrict__ H, const int* __restrict__ pos,
+                                            double* __restrict__ sH, float* __restrict__ sHf, int max_sweeps, int gid,
+                                            double* lds)
 {
     using KI = KindInfo<KIND>;
     constexpr int N = KI::N, G = KI::G;
@@ -699,12 +724,17 @@ __device__ __forceinline__ void contact_row(int n, double* __restrict__ H, int m
         }
     }
     if (!act) return;
+    if (!pos) {
 #pragma unroll
-    for (int k = 0; k < N; k++) Hr[k] = out[k];
-    if (Hf) {  // FP32 copy for the FP32 iterations
-        float* Hfr = Hf + (size_t)r * N * N + (size_t)l * N;
+        for (int k = 0; k < N; k++) Hr[k] = out[k];
+        return;
+    }
+    const size_t e = 36 * (size_t)pos[KI::K * r + l / 3] + 3 * (l % 3);
 #pragma unroll
-        for (int k = 0; k < N; k++) Hfr[k] = (float)out[k];
+    for (int k = 0; k < N; k++) sH[e + 9 * (k / 3) + k % 3] = out[k];
+    if (sHf) {
+#pragma unroll
+        for (int k = 0; k < N; k++) sHf[e + 9 * (k / 3) + k % 3] = (float)out[k];
     }
 }
 
@@ -716,9 +746,10 @@ k_contact(ContactBatch cb, int max_sweeps)
     int b = (int)blockIdx.x, t = 0;
     while (t < NTYPES - 1 && b >= cb.boff[t + 1]) t++;
     int gid = (b - cb.boff[t]) * TPB + (int)threadIdx.x;
-#define CONTACT_CASE(K)                                                     \
-    case K:                                                                 \
-        contact_row<K>(cb.n[K], cb.H[K], max_sweeps, gid, lds, cb.Hf[K]); \
+#define CONTACT_CASE(K)                                                                                        \
+    case K:                                                                                                    \
+        contact_row<K>(cb.n[K], cb.H[K], cb.pos ? cb.pos + cb.soff[K] : nullptr, cb.sd.H, cb.sd.Hf, max_sweeps, \
+                       gid, lds);                                                                              \
         break;
     switch (t) {
         CONTACT_CASE(0)
@@ -756,9 +787,6 @@ static int contact_launch(ContactBatch& cb, const double* x, const double* x0, d
 // the per-type tables a slot decodes through
 struct ContactSlots {
     const int* rows[NTYPES];
-    const double* H[NTYPES];
-    const float* Hf[NTYPES];            // FP32 copies (FP32 iterations), or null
-    const unsigned char* c64[NTYPES];   // rows that keep their FP64 Hessian
     int soff[NTYPES + 1];               // first slot of each type
 };
 __device__ __forceinline__ void slot_decode(const ContactSlots& cs, int s, int& t, int& r, int& a)
@@ -789,11 +817,13 @@ __global__ void k_cv_heads(int S, int nv, const int* __restrict__ keys, int* hea
     head[i] = i < S && keys[i] != nv && (i == 0 || keys[i] != keys[i - 1]) ? 1 : 0;
 }
 // pos = exclusive scan of head: run u starts at slot index i with pos[i] = u
-__global__ void k_cv_compact(int S, int nv, const int* __restrict__ keys, const int* __restrict__ pos, int* vert,
-                             int* ptr, int* count)
+// (and place[s] = the sorted place of slot s)
+__global__ void k_cv_compact(int S, int nv, const int* __restrict__ keys, const int* __restrict__ slot,
+                             const int* __restrict__ pos, int* vert, int* ptr, int* count, int* place)
 {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= S) return;
+    place[slot[i]] = i;
     const int k = keys[i];
     if (k == nv) return;
     const bool head = i == 0 || keys[i - 1] != k;
@@ -813,8 +843,7 @@ __global__ void k_cv_compact(int S, int nv, const int* __restrict__ keys, const 
 // (CV_G lanes per vertex): rhs -= g (after the inertia term), the diagonal
 // block written whole (k_rhs_init cleared every vertex's)
 __global__ void __launch_bounds__(TPB) k_cv_gather(const int* __restrict__ count, const int* __restrict__ vert,
-                                                   const int* __restrict__ ptr, const int* __restrict__ slot,
-                                                   ContactSlots cs, const double* __restrict__ cgrad, double* rhs,
+                                                   const int* __restrict__ ptr, SlotData sd, double* rhs,
                                                    double* cdiag)
 {
     const int gid = blockIdx.x * blockDim.x + threadIdx.x;
@@ -825,13 +854,11 @@ __global__ void __launch_bounds__(TPB) k_cv_gather(const int* __restrict__ count
     for (int k = 0; k < 12; k++) acc[k] = 0.0;
     if (live) {
         for (int e = ptr[u] + l; e < ptr[u + 1]; e += CV_G) {
-            int sl = slot[e], t, r, a;
-            slot_decode(cs, sl, t, r, a);
-            const int N = kind_dofs(t);
+            const int a = (sd.meta[e] >> 4) & 3;
 #pragma unroll
             for (int i = 0; i < 3; i++) {
-                acc[i] += cgrad[3 * (size_t)sl + i];
-                const double* h = cs.H[t] + (size_t)r * N * N + (size_t)(3 * a + i) * N + 3 * a;
+                acc[i] += sd.g[3 * (size_t)e + i];
+                const double* h = sd.H + 36 * (size_t)e + 9 * a + 3 * i;
                 acc[3 + 3 * i] += h[0]; acc[4 + 3 * i] += h[1]; acc[5 + 3 * i] += h[2];
             }
         }
@@ -919,50 +946,47 @@ static inline int spmv_grid(int nv)
     int nb = std::min(groups, SPMV_MAXB);
     return std::max(8, (nb + 7) & ~7);
 }
-// the contact part of a product: the contact vertices with their slot lists
+// the contact part of a product: the contact vertices with their slots
 struct ContactSet {
-    ContactSlots sl;
+    SlotData sd;
     const int* count;   // number of contact vertices (device)
     const int* vert;
     const int* ptr;
-    const int* slot;
 };
 // lane l's share of (sum_r H_r p_r) at contact vertex u: the vertex's slots
-// l, l + CV_G, ..., each the product of the slot's three Hessian rows 3 a + i
-// with the row's points, added into s[3].  With Hf set (FP32 iterations) a
-// row uses its FP32 copy unless flagged in c64.
+// l, l + CV_G, ..., each the product of the slot's three Hessian rows with the
+// row's points, added into s[3].  With Hf set (FP32 iterations) a slot uses its
+// FP32 copy unless it keeps FP64.  The slots' data is contiguous and needs no
+// table but ptr: through slot numbers, row tables and per-type Hessians, a chain
+// of five dependent loads, a product on two cubes in contact (520 rows) took
+// 13.7 us against 9.2, and on 27 cubes of 16^3 (29,367 rows) 40.3 against 32.1.
 template <class V>
 __device__ __forceinline__ void contact_vertex_spmv(const ContactSet& cs, const V* __restrict__ p, int u, int l,
                                                     double* s)
 {
     for (int e = cs.ptr[u] + l; e < cs.ptr[u + 1]; e += CV_G) {
-        int t, r, a;
-        slot_decode(cs.sl, cs.slot[e], t, r, a);
-        const int K = kind_points(t), N = 3 * K;
-        const int* rw = cs.sl.rows[t] + K * r;
-        const size_t off = (size_t)r * N * N + (size_t)(3 * a) * N;
-        // point by point (static indices, guarded up to the widest row), so
-        // only one point's p and the three partial rows are live
-        const bool f32 = cs.sl.Hf[t] && !cs.sl.c64[t][r];
-        const float* hf = f32 ? cs.sl.Hf[t] + off : nullptr;
-        const double* hd = cs.sl.H[t] + off;
+        const int4 id = cs.sd.ids[e];
+        const int mt = cs.sd.meta[e], K = mt & 7;
+        const bool f32 = cs.sd.Hf && !(mt & SLOT_KEEP64);
+        const int w[4] = {id.x, id.y, id.z, id.w};
         double a0 = 0.0, a1 = 0.0, a2 = 0.0;
 #pragma unroll
         for (int b = 0; b < 4; b++) {
             if (b < K) {
-                const int w = rw[b];
-                const double p0 = (double)p[3 * w], p1 = (double)p[3 * w + 1], p2 = (double)p[3 * w + 2];
+                const double p0 = (double)p[3 * w[b]], p1 = (double)p[3 * w[b] + 1], p2 = (double)p[3 * w[b] + 2];
+                double h[9];
                 if (f32) {
-                    const float* h = hf + 3 * b;
-                    a0 += (double)h[0] * p0 + (double)h[1] * p1 + (double)h[2] * p2;
-                    a1 += (double)h[N] * p0 + (double)h[N + 1] * p1 + (double)h[N + 2] * p2;
-                    a2 += (double)h[2 * N] * p0 + (double)h[2 * N + 1] * p1 + (double)h[2 * N + 2] * p2;
+                    const float* q = cs.sd.Hf + 36 * (size_t)e + 9 * b;
+#pragma unroll
+                    for (int k = 0; k < 9; k++) h[k] = (double)q[k];
                 } else {
-                    const double* h = hd + 3 * b;
-                    a0 += h[0] * p0 + h[1] * p1 + h[2] * p2;
-                    a1 += h[N] * p0 + h[N + 1] * p1 + h[N + 2] * p2;
-                    a2 += h[2 * N] * p0 + h[2 * N + 1] * p1 + h[2 * N + 2] * p2;
+                    const double* q = cs.sd.H + 36 * (size_t)e + 9 * b;
+#pragma unroll
+                    for (int k = 0; k < 9; k++) h[k] = q[k];
                 }
+                a0 += h[0] * p0 + h[1] * p1 + h[2] * p2;
+                a1 += h[3] * p0 + h[4] * p1 + h[5] * p2;
+                a2 += h[6] * p0 + h[7] * p1 + h[8] * p2;
             }
         }
         s[0] += a0; s[1] += a1; s[2] += a2;
@@ -1527,9 +1551,10 @@ extern "C" int fipc_destroy(fipc_ctx* c)
     release(c->vcent);
     release(c->tile_meta); release(c->tile_tcode); release(c->tile_vcode); release(c->tile_ppos); release(c->tile_vpos);
     release(c->tile_pptr); release(c->tile_vptr); release(c->tile_bpart); release(c->tile_gpart);
-    for (int t = 0; t < NTYPES; t++) { release(c->rows[t]); release(c->cH[t]); release(c->cHf[t]); release(c->c64[t]); }
+    for (int t = 0; t < NTYPES; t++) { release(c->rows[t]); release(c->cH[t]); }
     release(c->cv_keys); release(c->cv_vals); release(c->cv_keys2); release(c->cv_slot); release(c->cv_head);
     release(c->cv_vert); release(c->cv_ptr); release(c->cv_count); release(c->cgrad);
+    release(c->cv_place); release(c->cv_ids); release(c->cv_meta); release(c->cv_H); release(c->cv_Hf);
     release(c->keys_pp); release(c->keys_pe); release(c->keys_tmp); release(c->counters); release(c->cub_tmp); release(c->cub_tmp2); release(c->rows_tmp);
     release(c->nuniq); release(c->cdiag); release(c->Minv); release(c->r); release(c->z); release(c->pp); release(c->q); release(c->qc);
     release(c->Minvf); release(c->rf); release(c->zf); release(c->pf); release(c->qf);
@@ -1941,18 +1966,19 @@ extern "C" int fipc_residual(fipc_ctx* c, double* res)
 }
 
 // ---- assembly ----
-static ContactSlots contact_slots(fipc_ctx* c, bool fp32)
+static ContactSlots contact_slots(fipc_ctx* c)
 {
     ContactSlots sl;
     for (int t = 0; t < NTYPES; t++) {
         sl.rows[t] = c->rows[t].p;
-        sl.H[t] = c->cH[t].p;
-        sl.Hf[t] = fp32 ? c->cHf[t].p : nullptr;
-        sl.c64[t] = fp32 ? c->c64[t].p : nullptr;
         sl.soff[t] = c->soff[t];
     }
     sl.soff[NTYPES] = c->soff[NTYPES];
     return sl;
+}
+static SlotData slot_data(fipc_ctx* c, bool fp32)
+{
+    return SlotData{c->cv_ids.p, c->cv_meta.p, c->cv_H.p, fp32 ? c->cv_Hf.p : nullptr, c->cgrad.p};
 }
 // the contact vertices of the current rows (see fipc_ctx): slot keys, a
 // stable radix sort by vertex, run heads, their scan and the compaction; no
@@ -1972,8 +1998,10 @@ static int build_contact_vertices(fipc_ctx* c, hipStream_t st)
     STCHK(ensure(c->cv_keys, S)); STCHK(ensure(c->cv_vals, S)); STCHK(ensure(c->cv_keys2, S));
     STCHK(ensure(c->cv_slot, S)); STCHK(ensure(c->cv_head, (size_t)S + 1));
     STCHK(ensure(c->cv_vert, S)); STCHK(ensure(c->cv_ptr, (size_t)S + 1));
+    STCHK(ensure(c->cv_place, S)); STCHK(ensure(c->cv_ids, S)); STCHK(ensure(c->cv_meta, S));
+    STCHK(ensure(c->cv_H, (size_t)S * 36));
     HIPCHK(hipMemsetAsync(c->cv_count.p, 0, 4, st));
-    k_cv_keys<<<nblk(S), TPB, 0, st>>>(S, contact_slots(c, false), c->dmask.p, c->nv, c->cv_keys.p, c->cv_vals.p);
+    k_cv_keys<<<nblk(S), TPB, 0, st>>>(S, contact_slots(c), c->dmask.p, c->nv, c->cv_keys.p, c->cv_vals.p);
     HIPCHK(hipGetLastError());
     unsigned bits = 1;
     while ((1u << bits) <= (unsigned)c->nv) bits++;  // keys up to nv
@@ -1992,33 +2020,31 @@ static int build_contact_vertices(fipc_ctx* c, hipStream_t st)
     b2 = c->cub_tmp2.cap;
     HIPCHK(rocprim::exclusive_scan(c->cub_tmp2.p, b2, c->cv_head.p, c->cv_head.p, 0, (size_t)S + 1,
                                    rocprim::plus<int>(), st));
-    k_cv_compact<<<nblk(S), TPB, 0, st>>>(S, c->nv, c->cv_keys2.p, c->cv_head.p, c->cv_vert.p, c->cv_ptr.p,
-                                         c->cv_count.p);
+    k_cv_compact<<<nblk(S), TPB, 0, st>>>(S, c->nv, c->cv_keys2.p, c->cv_slot.p, c->cv_head.p, c->cv_vert.p,
+                                         c->cv_ptr.p, c->cv_count.p, c->cv_place.p);
     HIPCHK(hipGetLastError());
     return FIPC_OK;
 }
 static int launch_contacts(fipc_ctx* c, hipStream_t st)
 {
     if (c->cv_version != c->cons_version) STCHK(build_contact_vertices(c, st));
+    const int S = c->soff[NTYPES];
+    if (!S) return FIPC_OK;
+    const bool fp32 = c->precision == 1;
+    if (fp32) STCHK(ensure(c->cv_Hf, (size_t)S * 36));
     ContactBatch cb;
     for (int t = 0; t < NTYPES; t++) {
         cb.rows[t] = c->rows[t].p;
         cb.H[t] = c->cH[t].p;
         cb.n[t] = c->count[t];
-        const int N = kind_dofs(t);
-        if (c->precision == 1) {
-            STCHK(ensure(c->cHf[t], (size_t)std::max(c->count[t], 1) * N * N));
-            STCHK(ensure(c->c64[t], (size_t)std::max(c->count[t], 1)));
-        }
-        cb.Hf[t] = c->precision == 1 ? c->cHf[t].p : nullptr;
-        cb.c64[t] = c->precision == 1 ? c->c64[t].p : nullptr;
-        cb.cgrad[t] = c->cgrad.p + 3 * (size_t)c->soff[t];
+        cb.soff[t] = c->soff[t];
     }
-    const int S = c->soff[NTYPES];
-    if (!S) return FIPC_OK;
+    cb.pos = c->cv_place.p;
+    cb.g = nullptr;
+    cb.sd = slot_data(c, fp32);
     STCHK(contact_launch(cb, c->x.p, c->x0.p, c->dHat2, c->kappa, nullptr, 1, st));
-    k_cv_gather<<<nblk((long)CV_G * S), TPB, 0, st>>>(c->cv_count.p, c->cv_vert.p, c->cv_ptr.p, c->cv_slot.p,
-                                              contact_slots(c, false), c->cgrad.p, c->rhs.p, c->cdiag.p);
+    k_cv_gather<<<nblk((long)CV_G * S), TPB, 0, st>>>(c->cv_count.p, c->cv_vert.p, c->cv_ptr.p, cb.sd,
+                                                      c->rhs.p, c->cdiag.p);
     HIPCHK(hipGetLastError());
     return FIPC_OK;
 }
@@ -2101,11 +2127,10 @@ extern "C" int fipc_assemble(fipc_ctx* c, int precision)
 // the slot count, sizes the grid; the lanes past the device count exit)
 static int spmv_contacts(fipc_ctx* c, ContactSet& cs, bool fp32 = false)
 {
-    cs.sl = contact_slots(c, fp32);
+    cs.sd = slot_data(c, fp32);
     cs.count = c->cv_count.p;
     cs.vert = c->cv_vert.p;
     cs.ptr = c->cv_ptr.p;
-    cs.slot = c->cv_slot.p;
     int nb = c->soff[NTYPES] ? nblk((long)CV_G * c->soff[NTYPES]) : 0;
     return (nb + 7) & ~7;
 }
@@ -2693,8 +2718,11 @@ extern "C" int fipc_batch_constraint(int type, int n, const double* x, const dou
     ContactBatch cb;
     for (int t = 0; t < NTYPES; t++) {
         cb.rows[t] = drows; cb.H[t] = dH; cb.n[t] = t == type ? n : 0;
-        cb.Hf[t] = nullptr; cb.c64[t] = nullptr; cb.cgrad[t] = dg;
+        cb.soff[t] = 0;
     }
+    cb.pos = nullptr;
+    cb.g = dg;
+    cb.sd = SlotData{};
     STCHK(contact_launch(cb, dx, dx0, dHat2, kappa, dE, project, nullptr));
     HIPCHK(hipDeviceSynchronize());
     if (E) HIPCHK(hipMemcpy(E, dE, (size_t)n * 8, hipMemcpyDeviceToHost));
