@@ -168,6 +168,7 @@ struct fipc_ctx {
     size_t cub_bytes = 0;
     DVec<int> nuniq;
     // preconditioner + PCG
+    DVec<unsigned char> cgmask;  // per vertex: bit 0 Dirichlet, bit 1 contact vertex (of the last assembly)
     DVec<double> cdiag, Minv, r, z, pp, q, qc;   // q = A_bsr p, qc = contact part of A p
     // FP32 Hessian: the refinement rounds iterate on FP32 copies of the
     // preconditioner and of r, z, p, q (qc and the solution stay FP64)

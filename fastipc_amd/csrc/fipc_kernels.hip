@@ -406,7 +406,8 @@ constexpr int RHS_VPG = RHS_VPW * (TPB / 64);   // vertices per workgroup
 static inline int rhs_grid(long nv) { return (int)((nv + RHS_VPG - 1) / RHS_VPG); }
 __global__ void __launch_bounds__(TPB) k_rhs_init(int nv, const double* __restrict__ m, const double* __restrict__ x,
                                                   const double* __restrict__ xt,
-                                                  const unsigned char* __restrict__ dmask, double* rhs, double* cdiag)
+                                                  const unsigned char* __restrict__ dmask, double* rhs, double* cdiag,
+                                                  unsigned char* cgmask)
 {
     const int lane = threadIdx.x & 63;
     if (lane >= 3 * RHS_VPW) return;
@@ -414,6 +415,7 @@ __global__ void __launch_bounds__(TPB) k_rhs_init(int nv, const double* __restri
     const int d = lane % 3;
     if (i >= nv) return;
     for (int k = 0; k < 3; k++) cdiag[9 * i + 3 * d + k] = 0.0;
+    if (d == 0) cgmask[i] = dmask[i] ? 1 : 0;  // k_cv_gather marks the contact vertices
     rhs[3 * i + d] = dmask[i] ? 0.0 : -m[i] * (x[3 * i + d] - xt[3 * i + d]);
 }
 __global__ void __launch_bounds__(TPB) k_gather_tetg(int nv, const int* __restrict__ vcptr,
@@ -844,7 +846,7 @@ __global__ void k_cv_compact(int S, int nv, const int* __restrict__ keys, const 
 // block written whole (k_rhs_init cleared every vertex's)
 __global__ void __launch_bounds__(TPB) k_cv_gather(const int* __restrict__ count, const int* __restrict__ vert,
                                                    const int* __restrict__ ptr, SlotData sd, double* rhs,
-                                                   double* cdiag)
+                                                   double* cdiag, unsigned char* cgmask)
 {
     const int gid = blockIdx.x * blockDim.x + threadIdx.x;
     const int u = gid / CV_G, l = gid % CV_G;
@@ -875,6 +877,7 @@ __global__ void __launch_bounds__(TPB) k_cv_gather(const int* __restrict__ count
 #pragma unroll
     for (int k = 0; k < 3; k++) d[k] = i == 0 ? acc[3 + k] : (i == 1 ? acc[6 + k] : acc[9 + k]);
     rhs[3 * v + i] -= g;
+    if (i == 0) cgmask[v] = 2;
     cdiag[9 * v + 3 * i] = d[0]; cdiag[9 * v + 3 * i + 1] = d[1]; cdiag[9 * v + 3 * i + 2] = d[2];
 }
 
@@ -951,22 +954,28 @@ struct ContactSet {
     SlotData sd;
     const int* count;   // number of contact vertices (device)
     const int* vert;
-    const int* ptr;
+    const int* ptr;     // nslots + 1 entries, the first count + 1 set
+    int nslots;
 };
-// lane l's share of (sum_r H_r p_r) at contact vertex u: the vertex's slots
-// l, l + CV_G, ..., each the product of the slot's three Hessian rows with the
+// a lane's share of (sum_r H_r p_r) at a contact vertex: the slots e, e + CV_G,
+// ... below e1, each the product of the slot's three Hessian rows with the
 // row's points, added into s[3].  With Hf set (FP32 iterations) a slot uses its
 // FP32 copy unless it keeps FP64.  The slots' data is contiguous and needs no
 // table but ptr: through slot numbers, row tables and per-type Hessians, a chain
 // of five dependent loads, a product on two cubes in contact (520 rows) took
 // 13.7 us against 9.2, and on 27 cubes of 16^3 (29,367 rows) 40.3 against 32.1.
 template <class V>
-__device__ __forceinline__ void contact_vertex_spmv(const ContactSet& cs, const V* __restrict__ p, int u, int l,
+__device__ __forceinline__ void contact_vertex_spmv(const ContactSet& cs, const V* __restrict__ p, int e, int e1,
                                                     double* s)
 {
-    for (int e = cs.ptr[u] + l; e < cs.ptr[u + 1]; e += CV_G) {
-        const int4 id = cs.sd.ids[e];
-        const int mt = cs.sd.meta[e], K = mt & 7;
+    // the next slot's points are loaded while this one's product runs
+    int4 nid = make_int4(0, 0, 0, 0);
+    int nmt = 0;
+    if (e < e1) { nid = cs.sd.ids[e]; nmt = cs.sd.meta[e]; }
+    for (; e < e1; e += CV_G) {
+        const int4 id = nid;
+        const int mt = nmt, K = mt & 7;
+        if (e + CV_G < e1) { nid = cs.sd.ids[e + CV_G]; nmt = cs.sd.meta[e + CV_G]; }
         const bool f32 = cs.sd.Hf && !(mt & SLOT_KEEP64);
         const int w[4] = {id.x, id.y, id.z, id.w};
         double a0 = 0.0, a1 = 0.0, a2 = 0.0;
@@ -1000,7 +1009,9 @@ __global__ void __launch_bounds__(TPB) k_spmv(int nv, const int* __restrict__ ro
                                               const unsigned char* __restrict__ dmask, ContactSet cs, int nb_c,
                                               int nb_bsr, double* part, const int* __restrict__ state, int it)
 {
-    if (state && it > state[0]) return;
+    // the test that ends the launches queued past convergence is loaded with
+    // the first row bounds (slot bounds), not ahead of them
+    const int last = state ? state[0] : 0x7fffffff;
     double pq = 0.0;
     if ((int)blockIdx.x >= nb_c) {
         // the row groups are split into 8 contiguous ranges, one per XCD
@@ -1022,6 +1033,7 @@ __global__ void __launch_bounds__(TPB) k_spmv(int nv, const int* __restrict__ ro
         bool live = row < nv && g0 < g1;
         int nu0 = live ? rowptr[row] : 0, nu1 = live ? rowptr[row + 1] : 0;
         int nl0 = live ? lptr[row] : 0, nl1 = live ? lptr[row + 1] : 0;
+        if (it > last) return;
         for (int g = g0; g < g1; g += nbx) {
             row = g * SPMV_ROWS + rsub;
             int u0 = nu0, l0 = nl0;
@@ -1077,9 +1089,12 @@ __global__ void __launch_bounds__(TPB) k_spmv(int nv, const int* __restrict__ ro
         // butterfly; the sum is stored (each entry of qc has one writer)
         const int gid = (int)blockIdx.x * TPB + (int)threadIdx.x;
         const int u = gid / CV_G, l = gid % CV_G;
-        const bool live = u < cs.count[0];
+        const int n = cs.count[0];
+        const int e0 = u < cs.nslots ? cs.ptr[u] : 0, e1 = u < cs.nslots ? cs.ptr[u + 1] : 0;
+        if (it > last) return;
+        const bool live = u < n;
         double sv[3] = {0.0, 0.0, 0.0};
-        if (live) contact_vertex_spmv<V>(cs, p, u, l, sv);
+        if (live) contact_vertex_spmv<V>(cs, p, e0 + l, e1, sv);
 #pragma unroll
         for (int o = CV_G / 2; o > 0; o >>= 1) {
             sv[0] += __shfl_xor(sv[0], o, 64);
@@ -1109,7 +1124,7 @@ __global__ void __launch_bounds__(TPB) k_spmv(int nv, const int* __restrict__ ro
 // beforehand) becomes 0 if any increment is non-zero, so that the product
 // A x0 and its use can be skipped when x0 = 0 (then b - A x0 = b exactly)
 __global__ void k_pcg_x0(int nv, const double* xt, const double* xcur, const unsigned char* dmask, double* sol,
-                         double* qc, int* nonzero)
+                         int* nonzero)
 {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     bool nz = false;
@@ -1117,19 +1132,18 @@ __global__ void k_pcg_x0(int nv, const double* xt, const double* xcur, const uns
         for (int d = 0; d < 3; d++) {
             double v = dmask[i] ? xt[3 * i + d] - xcur[3 * i + d] : 0.0;
             sol[3 * i + d] = v;
-            qc[3 * i + d] = 0.0;
             nz |= v != 0.0;
         }
     }
     if (__ballot(nz) != 0 && (threadIdx.x & 63) == 0) nonzero[0] = 0;
 }
-// r = b - (q + qc) (= b - A x, from FP64 products); z = Minv r; p = z; qc
-// cleared for the iterations; partials of r.z and r.r.  V is the type the
+// r = b - (q + qc) (= b - A x, from FP64 products; qc only at contact vertices,
+// see k_pcg_cg's mask); z = Minv r; p = z; partials of r.z and r.r.  V is the type the
 // iterations keep r, z, p in (float for the FP32 Hessian's refinement rounds).
 // x0zero (may be null): -1 when x = 0, whose product was skipped (q, qc
 // not written: r = b)
 template <class V>
-__global__ void k_pcg_init(int nv, const double* b, const double* q, double* qc, const unsigned char* dmask,
+__global__ void k_pcg_init(int nv, const double* b, const double* q, const double* qc, const unsigned char* mask,
                            const double* Minv, V* r, V* z, V* p, double* part_rz, double* part_bb,
                            const int* x0zero)
 {
@@ -1138,14 +1152,14 @@ __global__ void k_pcg_init(int nv, const double* b, const double* q, double* qc,
     const bool skip = x0zero && x0zero[0] == -1;
     if (i < nv) {
         double ri[3], zi[3];
-        bool fixed = dmask[i];
+        const bool fixed = mask[i] & 1, touch = mask[i] & 2;
         for (int d = 0; d < 3; d++)
-            ri[d] = fixed ? 0.0 : (skip ? b[3 * i + d] : b[3 * i + d] - (q[3 * i + d] + qc[3 * i + d]));
+            ri[d] = fixed ? 0.0 : (skip ? b[3 * i + d] : b[3 * i + d] - (q[3 * i + d] + (touch ? qc[3 * i + d] : 0.0)));
         const double* M = Minv + 9 * i;
         for (int d = 0; d < 3; d++) zi[d] = fixed ? 0.0 : M[3 * d] * ri[0] + M[3 * d + 1] * ri[1] + M[3 * d + 2] * ri[2];
         for (int d = 0; d < 3; d++) {
             V rv = (V)ri[d], zv = (V)zi[d];
-            r[3 * i + d] = rv; z[3 * i + d] = zv; p[3 * i + d] = zv; qc[3 * i + d] = 0.0;
+            r[3 * i + d] = rv; z[3 * i + d] = zv; p[3 * i + d] = zv;
             rz += (double)rv * (double)zv;
             bb += ri[d] * ri[d];
         }
@@ -1226,34 +1240,87 @@ static inline int pcg_grid(int nv) { return std::min(nblk(nv), PCG_MAXB); }
 // so no block reads a value another block of the same launch writes.  One
 // launch replaces the two update kernels of the textbook form (whose second
 // waits for the r.z reduction of the first).
+//
+// The kernel is a chain of latencies, one vertex per thread on small meshes and
+// two at most (below 262,144 vertices), so everything is loaded before the first
+// wait: the state, the scalars, the partials of all three sums (reduced in one
+// pass, each in its own order) and the thread's first vertex.  In the order of
+// use, with a barrier pair per sum, it took 7.0 us on 2,008 vertices and 18.0 on
+// 110,600 in FP64, 6.5 on 24,695 and 14.5 on 200,016 in FP32; like this 4.6,
+// 14.0, 4.9 and 10.6 (200,016 vertices: 3.4 TB/s).
+// mask: bit 0 Dirichlet vertex, bit 1 contact vertex (whose product has a
+// contact part in qc; qc is read nowhere else).
 template <class V, class M>
-__global__ void __launch_bounds__(TPB) k_pcg_cg(int nv, double* scal, const unsigned char* __restrict__ dmask,
-                                                const M* __restrict__ Minv, V* __restrict__ u,
-                                                const V* __restrict__ w, double* __restrict__ qc,
-                                                V* __restrict__ p, V* __restrict__ s, V* __restrict__ x,
-                                                V* __restrict__ r, const double* part_uw, int nuw, double* part_g,
-                                                int npg, int* state, int it, double tol2)
+struct CgVertex {
+    V u[3], w[3], p[3], s[3], x[3], r[3];
+    M m[9];
+    unsigned char mask;
+};
+template <class V, class M>
+__device__ __forceinline__ void cg_load(CgVertex<V, M>& a, int i, bool first, const unsigned char* __restrict__ mask,
+                                        const M* __restrict__ Minv, const V* __restrict__ u, const V* __restrict__ w,
+                                        const V* __restrict__ p, const V* __restrict__ s, const V* __restrict__ x,
+                                        const V* __restrict__ r)
 {
-    if (it > state[0]) return;
-    const int cur = it & 1, prv = cur ^ 1;
-    double gamma, rr;
-    if (it == 0) {
-        gamma = scal[0];
-        rr = scal[4];
-    } else {
-        reduce_partials2(part_g + 2 * PCG_MAXB * prv, part_g + 2 * PCG_MAXB * prv + PCG_MAXB, npg, gamma, rr);
-        if (rr <= tol2 * scal[2] || !(rr == rr)) {
-            if (blockIdx.x == 0 && threadIdx.x == 0) {
-                state[0] = it - 1;
-                state[1] = it;
-                scal[4] = rr;
-            }
-            return;
-        }
+    const size_t k = 3 * (size_t)i;
+    a.mask = mask[i];
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+        a.u[d] = u[k + d];
+        a.w[d] = w[k + d];
+        a.x[d] = x[k + d];
+        a.r[d] = r[k + d];
+        a.p[d] = first ? (V)0 : p[k + d];
+        a.s[d] = first ? (V)0 : s[k + d];
     }
-    const double delta = reduce_partials(part_uw, nuw);
-    const double beta = it == 0 ? 0.0 : gamma / scal[6 + prv];
-    const double alpha = it == 0 ? gamma / delta : gamma / (delta - beta * gamma / scal[8 + prv]);
+#pragma unroll
+    for (int j = 0; j < 9; j++) a.m[j] = Minv[9 * (size_t)i + j];
+}
+template <class V, class M>
+__global__ void __launch_bounds__(TPB) k_pcg_cg(int nv, double* scal, const unsigned char* __restrict__ mask,
+                                                const M* __restrict__ Minv, V* __restrict__ u,
+                                                const V* __restrict__ w, const double* __restrict__ qc,
+                                                V* __restrict__ p, V* __restrict__ s, V* __restrict__ x,
+                                                V* __restrict__ r, const double* __restrict__ part_uw, int nuw,
+                                                double* part_g, int npg, int* state, int it, double tol2)
+{
+    const int cur = it & 1, prv = cur ^ 1;
+    const int last = state[0];
+    const double* pg = part_g + 2 * PCG_MAXB * prv;
+    double sd = 0.0, sg = 0.0, sr = 0.0;
+    for (int i = threadIdx.x; i < nuw; i += TPB) sd += part_uw[i];
+    if (it > 0)
+        for (int i = threadIdx.x; i < npg; i += TPB) { sg += pg[i]; sr += pg[PCG_MAXB + i]; }
+    const double rr0 = scal[2], gam0 = scal[0], res0 = scal[4], gprev = scal[6 + prv], aprev = scal[8 + prv];
+    int i = blockIdx.x * TPB + threadIdx.x;
+    CgVertex<V, M> a;
+    if (i < nv) cg_load(a, i, it == 0, mask, Minv, u, w, p, s, x, r);
+    if (it > last) return;
+    __shared__ double sh[3][TPB / 64];
+    sd = warp_sum(sd);
+    sg = warp_sum(sg);
+    sr = warp_sum(sr);
+    if ((threadIdx.x & 63) == 0) {
+        const int v = threadIdx.x >> 6;
+        sh[0][v] = sd; sh[1][v] = sg; sh[2][v] = sr;
+    }
+    __syncthreads();
+    double delta = 0.0, gamma = 0.0, rr = 0.0;
+#pragma unroll
+    for (int v = 0; v < TPB / 64; v++) { delta += sh[0][v]; gamma += sh[1][v]; rr += sh[2][v]; }
+    if (it == 0) {
+        gamma = gam0;
+        rr = res0;
+    } else if (rr <= tol2 * rr0 || !(rr == rr)) {
+        if (blockIdx.x == 0 && threadIdx.x == 0) {
+            state[0] = it - 1;
+            state[1] = it;
+            scal[4] = rr;
+        }
+        return;
+    }
+    const double beta = it == 0 ? 0.0 : gamma / gprev;
+    const double alpha = it == 0 ? gamma / delta : gamma / (delta - beta * gamma / aprev);
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         scal[6 + cur] = gamma;
         scal[8 + cur] = alpha;
@@ -1262,51 +1329,50 @@ __global__ void __launch_bounds__(TPB) k_pcg_cg(int nv, double* scal, const unsi
         state[1] = it + 1;
     }
     double ru = 0.0, rn2 = 0.0;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < nv; i += gridDim.x * blockDim.x) {
-        if (dmask[i]) continue;
-        // every load of the vertex is issued before the first store
-        const int k = 3 * i;
-        double uv[3], wv[3], qcv[3], pv[3], sv[3], xv[3], rv[3], Mi[9];
+    while (i < nv) {
+        const int in = i + gridDim.x * TPB;
+        CgVertex<V, M> b;
+        if (in < nv) cg_load(b, in, it == 0, mask, Minv, u, w, p, s, x, r);
+        if (!(a.mask & 1)) {
+            const size_t k = 3 * (size_t)i;
+            double qv[3] = {0.0, 0.0, 0.0}, ri[3];
+            if (a.mask & 2) { qv[0] = qc[k]; qv[1] = qc[k + 1]; qv[2] = qc[k + 2]; }
 #pragma unroll
-        for (int d = 0; d < 3; d++) {
-            uv[d] = (double)u[k + d];
-            wv[d] = (double)w[k + d];
-            qcv[d] = qc[k + d];
-            pv[d] = it == 0 ? 0.0 : (double)p[k + d];
-            sv[d] = it == 0 ? 0.0 : (double)s[k + d];
-            xv[d] = (double)x[k + d];
-            rv[d] = (double)r[k + d];
+            for (int d = 0; d < 3; d++) {
+                const V pn = (V)((double)a.u[d] + beta * (double)a.p[d]);
+                const V sn = (V)(((double)a.w[d] + qv[d]) + beta * (double)a.s[d]);
+                const V rn = (V)((double)a.r[d] - alpha * (double)sn);
+                p[k + d] = pn;
+                s[k + d] = sn;
+                x[k + d] = (V)((double)a.x[d] + alpha * (double)pn);
+                r[k + d] = rn;
+                ri[d] = (double)rn;
+            }
+#pragma unroll
+            for (int d = 0; d < 3; d++) {
+                const V un = (V)((double)a.m[3 * d] * ri[0] + (double)a.m[3 * d + 1] * ri[1] +
+                                 (double)a.m[3 * d + 2] * ri[2]);
+                u[k + d] = un;
+                ru += ri[d] * (double)un;
+                rn2 += ri[d] * ri[d];
+            }
         }
-#pragma unroll
-        for (int j = 0; j < 9; j++) Mi[j] = (double)Minv[9 * i + j];
-        double ri[3];
-#pragma unroll
-        for (int d = 0; d < 3; d++) {
-            // qc is non-zero only at contact vertices: cleared here, where
-            // it is consumed, for the next product
-            if (qcv[d] != 0.0) qc[k + d] = 0.0;
-            const V pn = (V)(uv[d] + beta * pv[d]);
-            const V sn = (V)((wv[d] + qcv[d]) + beta * sv[d]);
-            p[k + d] = pn;
-            s[k + d] = sn;
-            x[k + d] = (V)(xv[d] + alpha * (double)pn);
-            const V rnv = (V)(rv[d] - alpha * (double)sn);
-            r[k + d] = rnv;
-            ri[d] = (double)rnv;
-        }
-#pragma unroll
-        for (int d = 0; d < 3; d++) {
-            const V un = (V)(Mi[3 * d] * ri[0] + Mi[3 * d + 1] * ri[1] + Mi[3 * d + 2] * ri[2]);
-            u[k + d] = un;
-            ru += ri[d] * (double)un;
-            rn2 += ri[d] * ri[d];
-        }
+        a = b;
+        i = in;
     }
-    ru = block_sum(ru);
-    rn2 = block_sum(rn2);
-    if (threadIdx.x == 0) {
-        part_g[2 * PCG_MAXB * cur + blockIdx.x] = ru;
-        part_g[2 * PCG_MAXB * cur + PCG_MAXB + blockIdx.x] = rn2;
+    ru = warp_sum(ru);
+    rn2 = warp_sum(rn2);
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) {
+        const int v = threadIdx.x >> 6;
+        sh[0][v] = ru; sh[1][v] = rn2;
+    }
+    __syncthreads();
+    if (threadIdx.x < 2) {
+        double t = 0.0;
+#pragma unroll
+        for (int v = 0; v < TPB / 64; v++) t += sh[threadIdx.x][v];
+        part_g[2 * PCG_MAXB * cur + (threadIdx.x ? PCG_MAXB : 0) + blockIdx.x] = t;
     }
 }
 // the test of the last iteration's residual when the iteration budget ended
@@ -1556,7 +1622,7 @@ extern "C" int fipc_destroy(fipc_ctx* c)
     release(c->cv_vert); release(c->cv_ptr); release(c->cv_count); release(c->cgrad);
     release(c->cv_place); release(c->cv_ids); release(c->cv_meta); release(c->cv_H); release(c->cv_Hf);
     release(c->keys_pp); release(c->keys_pe); release(c->keys_tmp); release(c->counters); release(c->cub_tmp); release(c->cub_tmp2); release(c->rows_tmp);
-    release(c->nuniq); release(c->cdiag); release(c->Minv); release(c->r); release(c->z); release(c->pp); release(c->q); release(c->qc);
+    release(c->nuniq); release(c->cgmask); release(c->cdiag); release(c->Minv); release(c->r); release(c->z); release(c->pp); release(c->q); release(c->qc);
     release(c->Minvf); release(c->rf); release(c->zf); release(c->pf); release(c->qf);
     release(c->cgs); release(c->cgsf); release(c->part_g); release(c->dxf);
     release(c->trow); release(c->tval);
@@ -1773,7 +1839,7 @@ extern "C" int fipc_upload_mesh(fipc_ctx* c, int nv, const double* x0, const dou
     STCHK(ensure(c->x, n3)); STCHK(ensure(c->xn, n3)); STCHK(ensure(c->xt, n3)); STCHK(ensure(c->xprev, n3));
     STCHK(ensure(c->v, n3)); STCHK(ensure(c->sol, n3)); STCHK(ensure(c->rhs, n3)); STCHK(ensure(c->target, n3));
     STCHK(ensure(c->r, n3)); STCHK(ensure(c->z, n3)); STCHK(ensure(c->pp, n3)); STCHK(ensure(c->q, n3)); STCHK(ensure(c->qc, n3));
-    STCHK(ensure(c->cdiag, (size_t)nv * 9)); STCHK(ensure(c->Minv, (size_t)nv * 9));
+    STCHK(ensure(c->cdiag, (size_t)nv * 9)); STCHK(ensure(c->Minv, (size_t)nv * 9)); STCHK(ensure(c->cgmask, nv));
     HIPCHK(hipMemcpyAsync(c->x.p, x0, n3 * 8, hipMemcpyHostToDevice, c->s));
     c->x_version++;
     c->sys_version++;
@@ -2044,7 +2110,7 @@ static int launch_contacts(fipc_ctx* c, hipStream_t st)
     cb.sd = slot_data(c, fp32);
     STCHK(contact_launch(cb, c->x.p, c->x0.p, c->dHat2, c->kappa, nullptr, 1, st));
     k_cv_gather<<<nblk((long)CV_G * S), TPB, 0, st>>>(c->cv_count.p, c->cv_vert.p, c->cv_ptr.p, cb.sd,
-                                                      c->rhs.p, c->cdiag.p);
+                                                      c->rhs.p, c->cdiag.p, c->cgmask.p);
     HIPCHK(hipGetLastError());
     return FIPC_OK;
 }
@@ -2068,7 +2134,8 @@ extern "C" int fipc_assemble(fipc_ctx* c, int precision)
     // the tet pass and the block gather fill the GPU: the second stream
     // starts after the inertia term and the cleared diagonal blocks, and the
     // first waits for it before the tet gradients and the preconditioner
-    k_rhs_init<<<rhs_grid(c->nv), TPB, 0, c->s>>>(c->nv, c->m.p, c->x.p, c->xt.p, c->dmask.p, c->rhs.p, c->cdiag.p);
+    k_rhs_init<<<rhs_grid(c->nv), TPB, 0, c->s>>>(c->nv, c->m.p, c->x.p, c->xt.p, c->dmask.p, c->rhs.p, c->cdiag.p,
+                                                   c->cgmask.p);
     HIPCHK(hipGetLastError());
     HIPCHK(hipEventRecord(c->ev_rhs, c->s));
     HIPCHK(hipStreamWaitEvent(c->s2, c->ev_rhs, 0));
@@ -2131,11 +2198,12 @@ static int spmv_contacts(fipc_ctx* c, ContactSet& cs, bool fp32 = false)
     cs.count = c->cv_count.p;
     cs.vert = c->cv_vert.p;
     cs.ptr = c->cv_ptr.p;
+    cs.nslots = c->soff[NTYPES];
     int nb = c->soff[NTYPES] ? nblk((long)CV_G * c->soff[NTYPES]) : 0;
     return (nb + 7) & ~7;
 }
-// q + qc = A p (q = BSR part, qc = contact part accumulated: qc must be zero
-// on entry); prec selects the FP32 copy of the BSR values, V the type of p, q
+// q + qc = A p (q = BSR part; qc = contact part, stored at the contact vertices
+// only); prec selects the FP32 copy of the BSR values, V the type of p, q
 template <class V>
 static int spmv(fipc_ctx* c, int prec, const V* p, V* q, double* qc, double* part, const int* state, int it)
 {
@@ -2232,7 +2300,7 @@ static int pcg_round(fipc_ctx* c, int prec, const M* Minv, V* r, V* z, V* p, V* 
         // round 0 the product exits at once when x0 = 0 (the flag is -1)
         const int* x0zero = round == 0 ? c->x0flag.p : nullptr;
         STCHK(spmv<double>(c, c->precision, c->sol.p, c->q.p, c->qc.p, nullptr, x0zero, 0));
-        k_pcg_init<V><<<nbv, TPB, 0, c->s>>>(nv, c->rhs.p, c->q.p, c->qc.p, c->dmask.p, c->Minv.p, r, z, p,
+        k_pcg_init<V><<<nbv, TPB, 0, c->s>>>(nv, c->rhs.p, c->q.p, c->qc.p, c->cgmask.p, c->Minv.p, r, z, p,
                                              c->part_a.p, c->part_b.p, x0zero);
         HIPCHK(hipGetLastError());
         k_pcg_scalars<<<1, TPB, 0, c->s>>>(c->part_a.p, c->part_b.p, nbv, c->scal.p, c->pcg_state.p, round > 0, tol2);
@@ -2277,7 +2345,7 @@ static int pcg_round(fipc_ctx* c, int prec, const M* Minv, V* r, V* z, V* p, V* 
         for (; it < end; it++) {
             STCHK(spmv<V>(c, prec, z, q, c->qc.p, c->part_c.p, c->pcg_state.p, it));
             STCHK(fipc_tm_begin(c, TM_PCGVEC));
-            k_pcg_cg<V, M><<<nu, TPB, 0, c->s>>>(nv, c->scal.p, c->dmask.p, Minv, z, q, c->qc.p, p, sv, xs, r,
+            k_pcg_cg<V, M><<<nu, TPB, 0, c->s>>>(nv, c->scal.p, c->cgmask.p, Minv, z, q, c->qc.p, p, sv, xs, r,
                                                  c->part_c.p, nsp, c->part_g.p, nu, c->pcg_state.p, it, tol_it);
             STCHK(fipc_tm_end(c, TM_PCGVEC));
         }
@@ -2368,10 +2436,8 @@ static int solve_rounds(fipc_ctx* c, int first_round, double tol, int maxit, int
             // x0 = prescribed Dirichlet increments
             STCHK(ensure(c->x0flag, 1));
             HIPCHK(hipMemsetAsync(c->x0flag.p, 0xff, 4, c->s));
-            k_pcg_x0<<<nbv, TPB, 0, c->s>>>(nv, c->xt.p, c->x.p, c->dmask.p, c->sol.p, c->qc.p, c->x0flag.p);
+            k_pcg_x0<<<nbv, TPB, 0, c->s>>>(nv, c->xt.p, c->x.p, c->dmask.p, c->sol.p, c->x0flag.p);
             HIPCHK(hipGetLastError());
-        } else {
-            HIPCHK(hipMemsetAsync(c->qc.p, 0, (size_t)nv * 24, c->s));
         }
         int budget = maxit - total;
         // first chunk: the last first round's count, or that of the last
