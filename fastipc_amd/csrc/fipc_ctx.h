@@ -98,6 +98,7 @@ struct KernelTimer {
 struct fipc_ctx {
     hipStream_t s = nullptr;
     int nv = 0, nt = 0, nbp = 0, nbe = 0, nbt = 0, ndir = 0;
+    int nsurf = 0;  // vertices of the surface primitives
     // mesh
     DVec<int> tets, bp, be, bt, dids;
     DVec<double> IB, vol, la, mu, m;

@@ -1001,26 +1001,29 @@ __device__ __forceinline__ void contact_vertex_spmv(const ContactSet& cs, const 
         s[0] += a0; s[1] += a1; s[2] += a2;
     }
 }
+// nl_c blocks run the contact vertices.  Their partials take the first nb_c
+// places (an upper bound from the number of slots, which fixes the order of the
+// sum), the BSR blocks' those after; the places of the contact blocks that are
+// not launched, or have no vertices, are not read.
 template <class T, class V>
-__global__ void __launch_bounds__(TPB) k_spmv(int nv, const int* __restrict__ rowptr, const int* __restrict__ col,
-                                              const int* __restrict__ lptr, const int2* __restrict__ lent,
-                                              const T* __restrict__ val, const V* __restrict__ p,
-                                              V* __restrict__ q, double* qc,
-                                              const unsigned char* __restrict__ dmask, ContactSet cs, int nb_c,
-                                              int nb_bsr, double* part, const int* __restrict__ state, int it)
+__global__ void __launch_bounds__(TPB)
+k_spmv(int nv, const int* __restrict__ rowptr, const int* __restrict__ col, const int* __restrict__ lptr,
+       const int2* __restrict__ lent, const T* __restrict__ val, const V* __restrict__ p, V* __restrict__ q,
+       double* qc, const unsigned char* __restrict__ dmask, ContactSet cs, int nl_c, int nb_c, int nb_bsr,
+       double* part, const int* __restrict__ state, int it)
 {
     // the test that ends the launches queued past convergence is loaded with
     // the first row bounds (slot bounds), not ahead of them
     const int last = state ? state[0] : 0x7fffffff;
     double pq = 0.0;
-    if ((int)blockIdx.x >= nb_c) {
+    if ((int)blockIdx.x >= nl_c) {
         // the row groups are split into 8 contiguous ranges, one per XCD
         // (blocks are dispatched to XCDs round-robin); the XCD's blocks
         // interleave over its range, so at any time they cover consecutive
         // rows and the transposed blocks a row needs (stored up to a few
         // thousand rows above it) were read into the XCD's L2 by the sweep
         // just before
-        int bb = (int)blockIdx.x - nb_c;
+        int bb = (int)blockIdx.x - nl_c;
         int nbx = nb_bsr >> 3;
         int groups = (nv + SPMV_ROWS - 1) / SPMV_ROWS;
         int gpx = (groups + 7) >> 3;
@@ -1110,7 +1113,7 @@ __global__ void __launch_bounds__(TPB) k_spmv(int nv, const int* __restrict__ ro
     }
     if (part) {
         pq = block_sum(pq);
-        if (threadIdx.x == 0) part[blockIdx.x] = pq;
+        if (threadIdx.x == 0) part[(int)blockIdx.x < nl_c ? (int)blockIdx.x : (int)blockIdx.x - nl_c + nb_c] = pq;
     }
 }
 
@@ -1281,14 +1284,28 @@ __global__ void __launch_bounds__(TPB) k_pcg_cg(int nv, double* scal, const unsi
                                                 const M* __restrict__ Minv, V* __restrict__ u,
                                                 const V* __restrict__ w, const double* __restrict__ qc,
                                                 V* __restrict__ p, V* __restrict__ s, V* __restrict__ x,
-                                                V* __restrict__ r, const double* __restrict__ part_uw, int nuw,
-                                                double* part_g, int npg, int* state, int it, double tol2)
+                                                V* __restrict__ r, const double* __restrict__ part_uw, int nbc,
+                                                int nuw, const int* __restrict__ ncv, double* part_g, int npg,
+                                                int* state, int it, double tol2)
 {
     const int cur = it & 1, prv = cur ^ 1;
     const int last = state[0];
     const double* pg = part_g + 2 * PCG_MAXB * prv;
     double sd = 0.0, sg = 0.0, sr = 0.0;
-    for (int i = threadIdx.x; i < nuw; i += TPB) sd += part_uw[i];
+    // the product's partials: all, or (ncv set) those of the contact blocks that
+    // have vertices, then those of the BSR blocks (nbc .. nuw), loaded first
+    constexpr int NB = SPMV_MAXB / TPB + 1;
+    double db[NB], c0 = 0.0;
+    int used = 0;
+    if (ncv) {
+        used = min(nbc, (ncv[0] * CV_G + TPB - 1) / TPB);
+        c0 = part_uw[threadIdx.x];  // nbc > TPB
+        const int b0 = (int)threadIdx.x + (nbc - (int)threadIdx.x + TPB - 1) / TPB * TPB;
+#pragma unroll
+        for (int k = 0; k < NB; k++) db[k] = b0 + k * TPB < nuw ? part_uw[b0 + k * TPB] : 0.0;
+    } else {
+        for (int i = threadIdx.x; i < nuw; i += TPB) sd += part_uw[i];
+    }
     if (it > 0)
         for (int i = threadIdx.x; i < npg; i += TPB) { sg += pg[i]; sr += pg[PCG_MAXB + i]; }
     const double rr0 = scal[2], gam0 = scal[0], res0 = scal[4], gprev = scal[6 + prv], aprev = scal[8 + prv];
@@ -1296,6 +1313,12 @@ __global__ void __launch_bounds__(TPB) k_pcg_cg(int nv, double* scal, const unsi
     CgVertex<V, M> a;
     if (i < nv) cg_load(a, i, it == 0, mask, Minv, u, w, p, s, x, r);
     if (it > last) return;
+    if (ncv) {
+        if ((int)threadIdx.x < used) sd += c0;
+        for (int j = threadIdx.x + TPB; j < used; j += TPB) sd += part_uw[j];
+#pragma unroll
+        for (int k = 0; k < NB; k++) sd += db[k];
+    }
     __shared__ double sh[3][TPB / 64];
     sd = warp_sum(sd);
     sg = warp_sum(sg);
@@ -1873,6 +1896,18 @@ extern "C" int fipc_upload_mesh(fipc_ctx* c, int nv, const double* x0, const dou
     }
     c->cons_version++;  // no rows (and a new Dirichlet mask) from here
     {
+        // vertices of surface primitives: only these can be contact vertices
+        std::vector<char> on(nv, 0);
+        auto mark = [&](const int* v, int n) {
+            for (int i = 0; i < n; i++)
+                if (v[i] >= 0 && v[i] < nv) on[v[i]] = 1;
+        };
+        mark(bp, nbp);
+        mark(be, 2 * nbe);
+        mark(bt, 3 * nbt);
+        c->nsurf = (int)std::count(on.begin(), on.end(), 1);
+    }
+    {
         double mmin = 0.0;
         for (int i = 0; i < nv; i++)
             if (!dirichlet[i] && (mmin == 0.0 || m[i] < mmin)) mmin = m[i];
@@ -2202,6 +2237,25 @@ static int spmv_contacts(fipc_ctx* c, ContactSet& cs, bool fp32 = false)
     int nb = c->soff[NTYPES] ? nblk((long)CV_G * c->soff[NTYPES]) : 0;
     return (nb + 7) & ~7;
 }
+// contact blocks that a product launches, of the nbc that the slots would fill:
+// contact vertices are surface vertices, so the blocks past those have none (a
+// multiple of 8, so that a BSR block's XCD is that of its own index).  27 cubes
+// of 16^3, 29,367 rows: 1,144 instead of 3,352 blocks, 32.1 -> 31.1 us a product
+// and, with their partials left out, 14.0 -> 10.3 us an update.  Up to one
+// partial per thread of the update (two cubes, 520 rows: 72 blocks) all are
+// launched and read: 4.6 us an update against 5.0 with the test.
+static int contact_launched(const fipc_ctx* c, int nbc)
+{
+    return nbc <= TPB ? nbc : std::min(nbc, (nblk((long)CV_G * c->nsurf) + 7) & ~7);
+}
+template <class T, class V>
+static void spmv_launch(fipc_ctx* c, const T* val, const V* p, V* q, double* qc, const ContactSet& cs, int nbc, int nbb,
+                        double* part, const int* state, int it)
+{
+    const int nbl = contact_launched(c, nbc);
+    k_spmv<T, V><<<nbl + nbb, TPB, 0, c->s>>>(c->nv, c->rowptr.p, c->col.p, c->lptr.p, (const int2*)c->lent.p, val, p,
+                                              q, qc, c->dmask.p, cs, nbl, nbc, nbb, part, state, it);
+}
 // q + qc = A p (q = BSR part; qc = contact part, stored at the contact vertices
 // only); prec selects the FP32 copy of the BSR values, V the type of p, q
 template <class V>
@@ -2219,11 +2273,9 @@ static int spmv(fipc_ctx* c, int prec, const V* p, V* q, double* qc, double* par
     const int timer = part ? TM_SPMV : TM_SPMV_RES;
     STCHK(fipc_tm_begin(c, timer));
     if (prec == 1)
-        k_spmv<float, V><<<nbc + nbb, TPB, 0, c->s>>>(c->nv, c->rowptr.p, c->col.p, c->lptr.p, (const int2*)c->lent.p,
-                                                      c->valf.p, p, q, qc, c->dmask.p, cs, nbc, nbb, part, state, it);
+        spmv_launch<float, V>(c, c->valf.p, p, q, qc, cs, nbc, nbb, part, state, it);
     else
-        k_spmv<double, V><<<nbc + nbb, TPB, 0, c->s>>>(c->nv, c->rowptr.p, c->col.p, c->lptr.p, (const int2*)c->lent.p,
-                                                       c->val.p, p, q, qc, c->dmask.p, cs, nbc, nbb, part, state, it);
+        spmv_launch<double, V>(c, c->val.p, p, q, qc, cs, nbc, nbb, part, state, it);
     HIPCHK(hipGetLastError());
     STCHK(fipc_tm_end(c, timer));
     return FIPC_OK;
@@ -2280,6 +2332,8 @@ static int pcg_round(fipc_ctx* c, int prec, const M* Minv, V* r, V* z, V* p, V* 
                      double tol2, int hint, int state[2], bool reuse, bool* init_only, bool* cert_stop)
 {
     const int nv = c->nv, nbv = nblk(nv), nsp = spmv_nparts(c), nu = pcg_grid(nv), chunk = PCG_CHUNK;
+    const int nbc = nsp - spmv_grid(nv);
+    const int* ncv = contact_launched(c, nbc) < nbc ? c->cv_count.p : nullptr;
     const double tol_it = prec == 1 ? tol2 * (PCG_FP32_INNER * PCG_FP32_INNER) : tol2;
     V* sv = sizeof(V) == 4 ? (V*)(void*)c->cgsf.p : (V*)(void*)c->cgs.p;
     // the iterations' x: the FP64 solution, or the FP32 round's correction
@@ -2346,7 +2400,8 @@ static int pcg_round(fipc_ctx* c, int prec, const M* Minv, V* r, V* z, V* p, V* 
             STCHK(spmv<V>(c, prec, z, q, c->qc.p, c->part_c.p, c->pcg_state.p, it));
             STCHK(fipc_tm_begin(c, TM_PCGVEC));
             k_pcg_cg<V, M><<<nu, TPB, 0, c->s>>>(nv, c->scal.p, c->cgmask.p, Minv, z, q, c->qc.p, p, sv, xs, r,
-                                                 c->part_c.p, nsp, c->part_g.p, nu, c->pcg_state.p, it, tol_it);
+                                                 c->part_c.p, nbc, nsp, ncv, c->part_g.p, nu,
+                                                 c->pcg_state.p, it, tol_it);
             STCHK(fipc_tm_end(c, TM_PCGVEC));
         }
         HIPCHK(hipGetLastError());

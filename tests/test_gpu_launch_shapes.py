@@ -36,3 +36,54 @@ def test_contact_rows_do_not_depend_on_their_number(kind):
         part = _constraints(kind, X[:n].copy(), X0[:n].copy())
         for a, b in zip(part, whole):
             assert np.array_equal(a, b[:n], equal_nan=True), n
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("shape", [(1, 1, 3), (2, 3, 5), (3, 4, 9)])  # contact slots in one, many, and more blocks than surface vertices fill
+def test_product_and_solve_with_contacts(shape, precision):
+    """The product's contact part and the solver on piles whose contact blocks
+    fit one partial per thread, and on one whose slots would fill more blocks
+    than its surface vertices: the solution's residual by the product itself."""
+    import ctypes as C
+    from fastipc_amd import scene as S
+    from fastipc_amd.newton import NewtonIPC
+    m, layers, n = shape
+    xc, tc = S.lattice(n)
+    edge = (n - 1) * S.LATTICE_SPACING
+    xs, ts, nv = [], [], 0
+    for layer in range(layers):
+        for i in range(m):
+            for k in range(m):
+                off = [(1.06 * i + 0.31 * (layer % 2)) * edge, layer * (edge + 1e-3) + 1e-3, (1.06 * k + 0.17 * (layer % 2)) * edge]
+                xs.append(xc + off)
+                ts.append(tc + nv)
+                nv += len(xc)
+    gx, gt = S.box([-edge, -0.1, -edge], [(m + 2) * edge, 0.0, (m + 2) * edge])
+    x, tets = np.concatenate(xs + [gx]), np.concatenate(ts + [gt + nv]).astype(np.int32)
+    one = np.ones(len(tets))
+    sc = S.Scene(name="pile", x=x, tets=tets, density=1000 * one, youngs=1e5 * one, poisson=0.4 * one,
+                 dirichlet_mask=np.arange(len(x)) >= nv, dt=0.01)
+    sim = NewtonIPC(sc, precision=precision)
+    rng = np.random.default_rng(n)
+    state = sc.x.copy()
+    state[:nv] += rng.uniform(-1e-4, 1e-4, (nv, 3))
+    sim.set_state(state, np.zeros_like(state))
+    sim.compute_xn_and_xTilde(0.0)
+    counts = sim.find_constraints()
+    assert sum(counts) > 0 and sim.check_collision() == 0
+    sim.compute_hessian_and_gradient()
+    tol = 1e-6
+    sim.solve_system(tol=tol)
+    assert sim.last_solve_converged
+    p, b, y = sim.vector(1), sim.vector(2), np.zeros((sim.nv, 3))
+    _lib.call("fipc_spmv", sim.ctx, _lib.dptr(p), _lib.dptr(y))
+    # the recurrence's residual met the tolerance; the true one is near it
+    assert np.linalg.norm(b - y) <= 2 * tol * np.linalg.norm(b)
+    # symmetric: u.(A v) = v.(A u) up to the rounding of sums of some thousand terms
+    u, v = rng.standard_normal((2, sim.nv, 3))
+    u[nv:] = v[nv:] = 0
+    yu, yv = np.zeros_like(y), np.zeros_like(y)
+    _lib.call("fipc_spmv", sim.ctx, _lib.dptr(u), _lib.dptr(yu))
+    _lib.call("fipc_spmv", sim.ctx, _lib.dptr(v), _lib.dptr(yv))
+    assert abs(np.vdot(u, yv) - np.vdot(v, yu)) <= 1e-9 * np.linalg.norm(u) * np.linalg.norm(yv)
+    sim.close()
