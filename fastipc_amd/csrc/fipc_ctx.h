@@ -64,6 +64,7 @@ static inline void release(DVec<T>& v)
 struct Grid {
     unsigned M = 0;        // bucket count (power of two, >= cap)
     int cap = 0;           // entry capacity; grows when a build overflows
+    DVec<float> ibox;      // per item: its box in single precision, rounded outward (8 floats)
     DVec<int> cnt;         // per item: first entry within its block of items (two-level offsets)
     DVec<int> part;        // per block of items: its entries; part[blocks] = all entries
     DVec<unsigned> ekey;   // bucket of each entry
@@ -71,6 +72,7 @@ struct Grid {
     DVec<unsigned long long> ecell, cells;  // exact cell key per entry / ordered by bucket
     DVec<int> bstart;      // M+1 bucket offsets (bucket ends after the scatter)
     DVec<int> items;       // entries ordered by bucket
+    DVec<int> qinfo;       // per query: its box, vertices and cell range (16 words)
     DVec<int> qoff, qpart; // query cell offsets within blocks of queries, per-block totals
     // what the grid holds, for reuse by a later operation: the x version,
     // primitive kind, count and inflation of a grid of boxes at x; for a grid

@@ -1653,7 +1653,7 @@ extern "C" int fipc_destroy(fipc_ctx* c)
     release(c->x0flag);
     release(c->epart); release(c->amin); release(c->flag);
     for (Grid& g : c->grid) {
-        release(g.cnt); release(g.ekey); release(g.eitem); release(g.bstart);
+        release(g.ibox); release(g.qinfo); release(g.cnt); release(g.ekey); release(g.eitem); release(g.bstart);
         release(g.items); release(g.ecell); release(g.cells); release(g.qoff); release(g.part); release(g.qpart);
     }
     release(c->ccd_pairs[0]); release(c->ccd_pairs[1]);

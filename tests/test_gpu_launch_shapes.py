@@ -87,3 +87,41 @@ def test_product_and_solve_with_contacts(shape, precision):
     _lib.call("fipc_spmv", sim.ctx, _lib.dptr(v), _lib.dptr(yv))
     assert abs(np.vdot(u, yv) - np.vdot(v, yu)) <= 1e-9 * np.linalg.norm(u) * np.linalg.norm(yv)
     sim.close()
+
+
+def _brute_pairs(x, sc, dhat):
+    """point-triangle and edge-edge pairs whose boxes overlap within dhat, without a common vertex"""
+    bp, be, bt = sc.boundary
+    lo, hi = x[bt].min(1), x[bt].max(1)
+    pt = ((x[bp][:, None] < hi[None] + dhat) & (lo[None] - dhat < x[bp][:, None])).all(2)
+    pt &= (bp[:, None, None] != bt[None]).all(2)
+    lo, hi = x[be].min(1), x[be].max(1)
+    ee = ((lo[:, None] < hi[None] + dhat) & (lo[None] - dhat < hi[:, None])).all(2)
+    ee &= (be[:, None, :, None] != be[None, :, None, :]).all((2, 3))
+    return int(pt.sum()), int(np.triu(ee, 1).sum())
+
+
+@pytest.mark.parametrize("n,copies,spread", [(2, 1, 1.0), (2, 3, 0.3), (3, 2, 0.2), (4, 9, 0.9), (5, 4, 0.4), (2, 40, 0.5)])
+def test_grid_queries_visit_every_pair_once(n, copies, spread):
+    """The pairs that the searches' queries visit, counted, against all pairs of
+    boxes: one wave's pairs, several blocks of queries, crowded and nearly empty
+    buckets, and the few large boxes of the ground among them."""
+    import ctypes as C
+    from fastipc_amd import scene as S
+    from fastipc_amd.newton import NewtonIPC
+    rng = np.random.default_rng(1000 * n + copies)
+    xc, tc = S.lattice(n)
+    xs = [xc + rng.uniform(0, spread, 3) + [0, 0.05, 0] for _ in range(copies)]
+    gx, gt = S.box([-1, -0.1, -1], [2, 0.0, 2])
+    x = np.concatenate(xs + [gx])
+    tets = np.concatenate([tc + k * len(xc) for k in range(copies)] + [gt + copies * len(xc)]).astype(np.int32)
+    one = np.ones(len(tets))
+    sc = S.Scene(name="crowd", x=x, tets=tets, density=1000 * one, youngs=1e5 * one, poisson=0.4 * one,
+                 dirichlet_mask=np.arange(len(x)) >= copies * len(xc), dt=0.01, dhat_rel=2e-2)
+    sim = NewtonIPC(sc)
+    moved = sc.x + rng.normal(0, 0.01, sc.x.shape)
+    sim.set_state(moved, np.zeros_like(moved))
+    sim.search_stats(True)
+    sim.find_constraints()
+    assert tuple(sim.search_counts()) == _brute_pairs(moved, sc, sc.dhat)
+    sim.close()
