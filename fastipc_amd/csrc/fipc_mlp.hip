@@ -164,17 +164,20 @@ __global__ void k_sum_slices(long n, int S, const float* P, float* out)
     for (int s = 0; s < S; s++) v += P[s * n + i];
     out[i] = v;
 }
-// column sums of A[M][N] (N <= 64 per block column group): out[c] = sum_m A[m][c]
-__global__ void k_colsum(int M, int N, const float* A, float* out)
+// column sums of slices of A[M][N]: out[z N + c] = sum of A[m][c] over the rows of
+// slice z = blockIdx.y
+__global__ void k_colsum(int M, int N, int slice, const float* A, float* out)
 {
     __shared__ float sh[4][64];
     int c = blockIdx.x * 64 + (threadIdx.x & 63), r0 = threadIdx.x >> 6;
+    int m0 = blockIdx.y * slice, m1 = min(M, m0 + slice);
     float v = 0.f;
     if (c < N)
-        for (int m = r0; m < M; m += 4) v += A[(long)m * N + c];
+        for (int m = m0 + r0; m < m1; m += 4) v += A[(long)m * N + c];
     sh[r0][threadIdx.x & 63] = v;
     __syncthreads();
-    if (r0 == 0 && c < N) out[c] = sh[0][threadIdx.x] + sh[1][threadIdx.x] + sh[2][threadIdx.x] + sh[3][threadIdx.x];
+    if (r0 == 0 && c < N)
+        out[(long)blockIdx.y * N + c] = sh[0][threadIdx.x] + sh[1][threadIdx.x] + sh[2][threadIdx.x] + sh[3][threadIdx.x];
 }
 // dY = 2 (Y - T) / (M N); per-block partial sums of (Y - T)^2 / (M N)
 __global__ void k_mse(long n, float inv, const float* Y, const float* T, float* dY, float* part)
@@ -368,13 +371,340 @@ k_mlp_infer(int n, const float* __restrict__ X, const __bf16* __restrict__ Wt, c
             for (int i = 0; i < 3; i++) Y[gr * 3 + i] = acc[0][0][i] + bias[i];
     }
 }
-// Wt (BF16, transposed, last layer padded to 32 rows) from the FP32 parameters
-__global__ void k_pack_wt(int fi, int fo, int rows, const float* __restrict__ W, __bf16* __restrict__ Wt)
+// BF16 weights of the warm-start shape from the FP32 parameters, one launch: per
+// layer Wt[n][k] (transposed, the last padded to 32 rows), then, for the
+// backward products, W[k][n] of layers 1 to 4 (the last padded to 16 columns)
+constexpr int FI_L = 5, FI_IN = 16, FI_OUT = 3;
+constexpr long FI_WT = (long)FI_W * FI_IN + 3L * FI_W * FI_W + 32L * FI_W;  // elements of the first part
+constexpr long FI_WN = 3L * FI_W * FI_W + 16L * FI_W;                       // and of the second
+__global__ void k_pack_weights(const float* __restrict__ params, const long* __restrict__ boff, __bf16* __restrict__ w,
+                               long total)
 {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= rows * fi) return;
-    int nrow = i / fi, k = i % fi;
-    Wt[i] = (__bf16)(nrow < fo ? W[(long)k * fo + nrow] : 0.f);
+    const long i = blockIdx.x * (long)blockDim.x + threadIdx.x;
+    if (i >= total) return;
+    long j = i;
+    float v = 0.f;
+    if (i < FI_WT) {
+        int l = 0;
+        long size = (long)FI_W * FI_IN;
+        while (j >= size) { j -= size; l++; size = l == FI_L - 1 ? 32L * FI_W : (long)FI_W * FI_W; }
+        const int fi = l == 0 ? FI_IN : FI_W, fo = l == FI_L - 1 ? FI_OUT : FI_W;
+        const int n = (int)(j / fi), k = (int)(j % fi);
+        if (n < fo) v = params[boff[l] - (long)fi * fo + (long)k * fo + n];
+    } else {
+        j -= FI_WT;
+        const int l = j < 3L * FI_W * FI_W ? 1 + (int)(j / (FI_W * FI_W)) : FI_L - 1;
+        j -= (l - 1L) * FI_W * FI_W;
+        const int fo = l == FI_L - 1 ? FI_OUT : FI_W, ld = l == FI_L - 1 ? 16 : FI_W;
+        const int k = (int)(j / ld), n = (int)(j % ld);
+        if (n < fo) v = params[boff[l] - (long)FI_W * fo + (long)k * fo + n];
+    }
+    w[i] = (__bf16)v;
+}
+
+// ---------------------------------------------------------------------------
+// Fused training for the warm-start shape, in three launches after the packing:
+//  - k_mlp_fwdbwd: a block takes 32 rows through the five layers and back.  A
+//    wave owns 64 features: their pre-activations stay in its registers (4 x 32
+//    floats), activations and gradients pass between waves through one LDS tile
+//    in BF16 (the precision of the products' inputs).  What the weight gradients
+//    need, the inputs A_l of the layers and the gradients G_l at their outputs, is
+//    written in BF16, transposed ([feature][row]), so that the next launch's
+//    fragments (8 consecutive rows of a feature) are 16-byte loads; the bias
+//    gradients' FP32 column sums and the loss are written per block;
+//  - k_mlp_dw: dW_l = A_l^T G_l in 64 x 64 tiles over row slices;
+//  - k_mlp_sum: the slices' and the blocks' sums.
+// Layer by layer, with FP32 activations in HBM and a column sum of 8,192 rows
+// in four workgroups (385 us a layer), loss and gradient of 8,192 rows took
+// 3.0 ms of kernels; like this 168 us.
+// ---------------------------------------------------------------------------
+struct TrainBufs {
+    __bf16* A;      // A_0 [16][ld], then A_1 .. A_4 [256][ld]
+    __bf16* G;      // G_0 .. G_3 [256][ld], then G_4 [32][ld]
+    float* bias;    // per block 4 x 256 + 3 column sums
+    float* loss;    // per block
+    long ld;        // rows, a multiple of 32
+};
+constexpr int FI_NB = 4 * FI_W + FI_OUT;  // bias parameters
+__device__ __forceinline__ long fi_a(int l, long ld) { return l == 0 ? 0 : (FI_IN + (l - 1L) * FI_W) * ld; }
+// D[feature][row] for this wave's 64 features of the block's 32 rows; four k
+// steps of weight fragments are in flight ahead of the products
+template <int KIN>
+__device__ __forceinline__ void ft_layer(const __bf16* __restrict__ W, const __bf16 (*H)[FI_LDS], int f0, int lane,
+                                         floatx16 (&acc)[2])
+{
+    constexpr int CH = KIN == 16 ? 1 : 4;  // k steps per chunk
+    const __bf16* wp[2];
+#pragma unroll
+    for (int f = 0; f < 2; f++) {
+        wp[f] = W + (long)(f0 + f * 32 + (lane & 31)) * KIN + (lane >> 5) * 8;
+#pragma unroll
+        for (int j = 0; j < 16; j++) acc[f][j] = 0.f;
+    }
+    bf16x8 a[2][CH], an[2][CH];
+#pragma unroll
+    for (int f = 0; f < 2; f++)
+#pragma unroll
+        for (int c = 0; c < CH; c++) a[f][c] = *(const bf16x8*)(wp[f] + 16 * c);
+#pragma unroll
+    for (int k0 = 0; k0 < KIN; k0 += 16 * CH) {
+        if (k0 + 16 * CH < KIN)
+#pragma unroll
+            for (int f = 0; f < 2; f++)
+#pragma unroll
+                for (int c = 0; c < CH; c++) an[f][c] = *(const bf16x8*)(wp[f] + k0 + 16 * (CH + c));
+#pragma unroll
+        for (int c = 0; c < CH; c++) {
+            const bf16x8 b = *(const bf16x8*)&H[lane & 31][k0 + 16 * c + (lane >> 5) * 8];
+#pragma unroll
+            for (int f = 0; f < 2; f++) acc[f] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[f][c], b, acc[f], 0, 0, 0);
+        }
+#pragma unroll
+        for (int f = 0; f < 2; f++)
+#pragma unroll
+            for (int c = 0; c < CH; c++) a[f][c] = an[f][c];
+    }
+}
+// value j of tile f of a lane belongs to feature f0 + 32 f + 8 (j / 4) + 4 (lane / 32)
+// + j % 4 of row lane % 32: to the LDS tile ([row][feature]) and, transposed, to
+// dst ([feature][ld])
+__device__ __forceinline__ void ft_store(const float (&v)[2][16], __bf16 (*H)[FI_LDS], __bf16* __restrict__ dst, long ld,
+                                         long r0, int f0, int lane)
+{
+#pragma unroll
+    for (int f = 0; f < 2; f++)
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+            const int m = f0 + 32 * f + 8 * g + 4 * (lane >> 5);
+            uint2 pk;
+            unsigned int b[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                b[i] = bf16_bits(v[f][4 * g + i]);
+                ((unsigned short*)dst)[(m + i) * ld + r0 + (lane & 31)] = (unsigned short)b[i];
+            }
+            pk.x = b[0] | (b[1] << 16);
+            pk.y = b[2] | (b[3] << 16);
+            *(uint2*)&H[lane & 31][m] = pk;
+        }
+}
+// column sums over the block's 32 rows: each step hands half of the values to the
+// lane across, so 31 exchanges reduce 32 values; lane l % 32 ends with value l % 32
+__device__ __forceinline__ void ft_colsum(const float (&v)[2][16], float* __restrict__ out, int f0, int lane)
+{
+    float w[32];
+#pragma unroll
+    for (int k = 0; k < 32; k++) w[k] = v[k >> 4][k & 15];
+#pragma unroll
+    for (int s = 16, n = 16; s > 0; s >>= 1, n >>= 1) {
+        const bool up = lane & s;
+#pragma unroll
+        for (int k = 0; k < n; k++) {
+            const float send = up ? w[k] : w[k + n], keep = up ? w[k + n] : w[k];
+            w[k] = keep + __shfl_xor(send, s, 64);
+        }
+    }
+    const int k = lane & 31, j = k & 15;
+    out[f0 + 32 * (k >> 4) + 8 * (j >> 2) + 4 * (lane >> 5) + (j & 3)] = w[0];
+}
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2)))
+k_mlp_fwdbwd(int n, const float* __restrict__ X, const float* __restrict__ T, const __bf16* __restrict__ Wt,
+             const float* __restrict__ params, const long* __restrict__ boff, float inv, TrainBufs tb)
+{
+    __shared__ __attribute__((aligned(16))) __bf16 H[32][FI_LDS];
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int f0 = w * 64;
+    const long r0 = (long)blockIdx.x * 32, ld = tb.ld;
+    const __bf16* Wn = Wt + FI_WT;
+    float* bias = tb.bias + (long)blockIdx.x * FI_NB;
+    for (int e = tid; e < 32 * FI_IN; e += 256) {
+        const int r = e >> 4, k = e & 15;
+        H[r][k] = (__bf16)(r0 + r < n ? X[(r0 + r) * FI_IN + k] : 0.f);
+    }
+    __syncthreads();
+    for (int e = tid; e < 32 * FI_IN; e += 256) tb.A[(long)(e >> 5) * ld + r0 + (e & 31)] = H[e & 31][e >> 5];
+    // forward
+    float z[4][2][16], v[2][16];
+    floatx16 acc[2];
+    const __bf16* W = Wt;
+#pragma unroll
+    for (int l = 0; l < 4; l++) {
+        if (l == 0) ft_layer<FI_IN>(W, H, f0, lane, acc);
+        else ft_layer<FI_W>(W, H, f0, lane, acc);
+        const float* b = params + boff[l];
+#pragma unroll
+        for (int f = 0; f < 2; f++)
+#pragma unroll
+            for (int j = 0; j < 16; j++) {
+                const float zz = acc[f][j] + b[f0 + 32 * f + 8 * (j >> 2) + 4 * (lane >> 5) + (j & 3)];
+                z[l][f][j] = zz;
+                v[f][j] = zz * sigm(zz);
+            }
+        __syncthreads();  // every wave has read this layer's input
+        ft_store(v, H, tb.A + fi_a(l + 1, ld), ld, r0, f0, lane);
+        __syncthreads();
+        W += (long)FI_W * (l == 0 ? FI_IN : FI_W);
+    }
+    // output layer (its first 32-feature tile, on the first wave): loss and G_4
+    float dy[3] = {0.f, 0.f, 0.f};
+    if (w == 0) {
+        floatx16 y[1][1];
+#pragma unroll
+        for (int j = 0; j < 16; j++) y[0][0][j] = 0.f;
+        fi_layer<FI_W, 1, 1>(W, H, 0, 0, lane, y);
+        const long gr = r0 + (lane & 31);
+        const float* b = params + boff[4];
+        float e = 0.f;
+        if (lane < 32 && gr < n)
+#pragma unroll
+            for (int i = 0; i < 3; i++) {
+                const float d = y[0][0][i] + b[i] - T[gr * 3 + i];
+                dy[i] = 2.f * d * inv;
+                e += d * d * inv;
+            }
+        float s[4] = {e, dy[0], dy[1], dy[2]};
+#pragma unroll
+        for (int o = 16; o > 0; o >>= 1)
+#pragma unroll
+            for (int i = 0; i < 4; i++) s[i] += __shfl_xor(s[i], o, 64);
+        if (lane == 0) {
+            tb.loss[blockIdx.x] = s[0];
+#pragma unroll
+            for (int i = 0; i < 3; i++) bias[4 * FI_W + i] = s[1 + i];
+        }
+    }
+    __syncthreads();
+    if (w == 0) {
+        // the gradient as the next product's input (16 columns, 3 used), and G_4
+        __bf16* g4 = tb.G + 4L * FI_W * ld;
+        if (lane < 32) {
+#pragma unroll
+            for (int k = 0; k < 16; k++) H[lane][k] = (__bf16)(k < 3 ? dy[k] : 0.f);
+#pragma unroll
+            for (int k = 0; k < 32; k++) g4[k * ld + r0 + lane] = (__bf16)(k < 3 ? dy[k] : 0.f);
+        }
+    }
+    __syncthreads();
+    // backward: G_{l-1} = (G_l W_l^T) silu'(z_{l-1})
+#pragma unroll
+    for (int l = 4; l >= 1; l--) {
+        const __bf16* B = Wn + (l - 1L) * FI_W * FI_W;
+        if (l == 4) ft_layer<16>(B, H, f0, lane, acc);
+        else ft_layer<FI_W>(B, H, f0, lane, acc);
+#pragma unroll
+        for (int f = 0; f < 2; f++)
+#pragma unroll
+            for (int j = 0; j < 16; j++) {
+                const float zz = z[l - 1][f][j], s = sigm(zz);
+                v[f][j] = acc[f][j] * (s * (1.f + zz * (1.f - s)));
+            }
+        __syncthreads();  // every wave has read G_l
+        ft_store(v, H, tb.G + (l - 1L) * FI_W * ld, ld, r0, f0, lane);
+        ft_colsum(v, bias + (l - 1) * FI_W, f0, lane);
+        __syncthreads();
+    }
+}
+// dW_l tiles: 64 inputs x 64 outputs of one layer over one slice of rows; the
+// four waves take every fourth k step and add their tiles in LDS in order.
+// Blocks of a slice: 4 tiles of layer 0 (16 inputs), 16 each of layers 1 to 3,
+// 4 of layer 4 (3 outputs)
+constexpr int FI_TILES = 4 + 3 * 16 + 4;
+__global__ void __launch_bounds__(256) k_mlp_dw(TrainBufs tb, int slice, const long* __restrict__ boff, long nparams,
+                                                float* __restrict__ part)
+{
+    __shared__ float S[64][65];
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int t = blockIdx.x;
+    const int l = t < 4 ? 0 : (t < 52 ? 1 + (t - 4) / 16 : 4);
+    const int fi = l == 0 ? FI_IN : FI_W, fo = l == 4 ? FI_OUT : FI_W, fog = l == 4 ? 32 : FI_W;
+    const int tt = t < 4 ? t : (t < 52 ? (t - 4) % 16 : t - 52);
+    const int m0 = l == 0 ? 0 : (l == 4 ? tt * 64 : (tt >> 2) * 64), n0 = l == 4 ? 0 : (l == 0 ? tt : tt & 3) * 64;
+    const long ld = tb.ld, k0 = (long)blockIdx.y * slice, k1 = min(ld, k0 + slice);
+    const __bf16* A = tb.A + fi_a(l, ld);
+    const __bf16* G = tb.G + (long)l * FI_W * ld;
+    floatx16 acc[2][2];
+#pragma unroll
+    for (int a = 0; a < 2; a++)
+#pragma unroll
+        for (int b = 0; b < 2; b++)
+#pragma unroll
+            for (int j = 0; j < 16; j++) acc[a][b][j] = 0.f;
+    const __bf16 *pa[2], *pb[2];
+    bool ina[2], inb[2];
+#pragma unroll
+    for (int a = 0; a < 2; a++) {
+        const int m = m0 + 32 * a + (lane & 31), c = n0 + 32 * a + (lane & 31);
+        ina[a] = m < fi;
+        inb[a] = c < fog;
+        pa[a] = A + (ina[a] ? m : 0) * ld + (lane >> 5) * 8;
+        pb[a] = G + (inb[a] ? c : 0) * ld + (lane >> 5) * 8;
+    }
+    bf16x8 zero;
+#pragma unroll
+    for (int i = 0; i < 8; i++) zero[i] = (__bf16)0.f;
+#pragma unroll 4
+    for (long k = k0 + 16 * w; k < k1; k += 64) {
+        bf16x8 fa[2], fb[2];
+#pragma unroll
+        for (int a = 0; a < 2; a++) {
+            fa[a] = ina[a] ? *(const bf16x8*)(pa[a] + k) : zero;
+            fb[a] = inb[a] ? *(const bf16x8*)(pb[a] + k) : zero;
+        }
+#pragma unroll
+        for (int a = 0; a < 2; a++)
+#pragma unroll
+            for (int b = 0; b < 2; b++)
+                acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[a], fb[b], acc[a][b], 0, 0, 0);
+    }
+    for (int v = 0; v < 4; v++) {
+        if (w == v)
+#pragma unroll
+            for (int a = 0; a < 2; a++)
+#pragma unroll
+                for (int b = 0; b < 2; b++)
+#pragma unroll
+                    for (int j = 0; j < 16; j++) {
+                        float& s = S[32 * a + 8 * (j >> 2) + 4 * (lane >> 5) + (j & 3)][32 * b + (lane & 31)];
+                        s = v == 0 ? acc[a][b][j] : s + acc[a][b][j];
+                    }
+        __syncthreads();
+    }
+    float* out = part + (long)blockIdx.y * nparams + boff[l] - (long)fi * fo;
+    for (int e = tid; e < 64 * 64; e += 256) {
+        const int m = m0 + (e >> 6), c = n0 + (e & 63);
+        if (m < fi && c < fo) out[(long)m * fo + c] = S[e >> 6][e & 63];
+    }
+}
+// grads: weights from S slices, biases from nb blocks' column sums (the first
+// nwb blocks take 64 biases each, 16 rows of threads over the blocks)
+__global__ void __launch_bounds__(1024) k_mlp_sum(long nparams, int S, const float* __restrict__ part, int nb,
+                                                  const float* __restrict__ bias, const long* __restrict__ boff,
+                                                  int nwb, float* __restrict__ grads)
+{
+    __shared__ float sh[16][64];
+    if ((int)blockIdx.x < nwb) {
+        const int c = (int)blockIdx.x * 64 + (threadIdx.x & 63), r = threadIdx.x >> 6;
+        float v = 0.f;
+        if (c < FI_NB)
+#pragma unroll 8
+            for (int b = r; b < nb; b += 16) v += bias[(long)b * FI_NB + c];
+        sh[r][threadIdx.x & 63] = v;
+        __syncthreads();
+        if (r == 0 && c < FI_NB) {
+            float t = 0.f;
+            for (int k = 0; k < 16; k++) t += sh[k][threadIdx.x];
+            grads[boff[min(c / FI_W, 4)] + (c < 4 * FI_W ? c % FI_W : c - 4 * FI_W)] = t;
+        }
+        return;
+    }
+    const long i = ((long)blockIdx.x - nwb) * 1024 + threadIdx.x;
+    if (i >= nparams) return;
+    for (int l = 0; l < FI_L; l++)
+        if (i >= boff[l] && i < boff[l] + (l == 4 ? FI_OUT : FI_W)) return;  // a bias
+    float v = 0.f;
+#pragma unroll 8
+    for (int s = 0; s < S; s++) v += part[s * nparams + i];
+    grads[i] = v;
 }
 
 // ---------------------------------------------------------------------------
@@ -396,6 +726,10 @@ struct fipc_mlp {
     bool fused = false;
     bool wt_ok = false;
     DVec<__bf16> wt;
+    // fused training: layer inputs and output gradients in BF16, transposed, and
+    // the blocks' bias sums
+    DVec<__bf16> tA, tG;
+    DVec<float> tbias;
     DVec<long> dboff;
     // dataset
     DVec<float> dsX, dsT;
@@ -406,17 +740,20 @@ struct fipc_mlp {
 static int mlp_reserve(fipc_mlp* m, int rows, bool train)
 {
     if (rows > m->cap) {
-        for (int l = 1; l <= m->L; l++) STCHK(ensure(m->H[l], (size_t)rows * m->dim[l]));
+        // the fused kernels keep the hidden layers on the chip
+        for (int l = m->fused ? m->L : 1; l <= m->L; l++) STCHK(ensure(m->H[l], (size_t)rows * m->dim[l]));
         m->cap = rows;
     }
     if (train && rows > m->tcap) {
-        for (int l = 1; l < m->L; l++) STCHK(ensure(m->Z[l], (size_t)rows * m->dim[l]));
-        int wmax = *std::max_element(m->dim.begin(), m->dim.end());
-        STCHK(ensure(m->dA, (size_t)rows * wmax));
-        STCHK(ensure(m->dB, (size_t)rows * wmax));
+        if (!m->fused) {
+            for (int l = 1; l < m->L; l++) STCHK(ensure(m->Z[l], (size_t)rows * m->dim[l]));
+            int wmax = *std::max_element(m->dim.begin(), m->dim.end());
+            STCHK(ensure(m->dA, (size_t)rows * wmax));
+            STCHK(ensure(m->dB, (size_t)rows * wmax));
+        }
         STCHK(ensure(m->X, (size_t)rows * m->n_in));
         STCHK(ensure(m->T, (size_t)rows * m->n_out));
-        STCHK(ensure(m->loss, (size_t)nblk((long)rows * m->n_out) + 8));
+        STCHK(ensure(m->loss, (size_t)std::max(nblk((long)rows * m->n_out), (rows + 31) / 32) + 8));
         m->tcap = rows;
     }
     return FIPC_OK;
@@ -440,17 +777,44 @@ static int mlp_forward(fipc_mlp* m, hipStream_t s, int n, const float* X, bool t
     return FIPC_OK;
 }
 
+static int mlp_pack(fipc_mlp* m, hipStream_t s);
+// loss partials of n rows: per block of the fused kernel, or of k_mse
+static int mlp_loss_parts(const fipc_mlp* m, int n) { return m->fused ? (n + 31) / 32 : nblk((long)n * m->n_out); }
+static int mlp_backward_fused(fipc_mlp* m, hipStream_t s, int n, const float* X, const float* T)
+{
+    const int nb = (n + 31) / 32;
+    // rows per slice of the weight gradients: at most 32 slices, of at least 256
+    // rows (a multiple of the four waves' 64)
+    const long ld = 32L * nb;
+    const int S = (int)std::max(1L, std::min(32L, ld / 512));
+    const int slice = (int)((ld + 64L * S - 1) / (64L * S)) * 64;
+    STCHK(mlp_pack(m, s));
+    STCHK(ensure(m->tA, (size_t)ld * (FI_IN + 4 * FI_W)));
+    STCHK(ensure(m->tG, (size_t)ld * (4 * FI_W + 32)));
+    STCHK(ensure(m->tbias, (size_t)nb * FI_NB));
+    STCHK(ensure(m->part, (size_t)S * m->nparams));
+    const TrainBufs tb{m->tA.p, m->tG.p, m->tbias.p, m->loss.p, ld};
+    k_mlp_fwdbwd<<<nb, 256, 0, s>>>(n, X, T, m->wt.p, m->params.p, m->dboff.p, 1.f / (float)((long)n * m->n_out), tb);
+    k_mlp_dw<<<dim3(FI_TILES, S), 256, 0, s>>>(tb, slice, m->dboff.p, m->nparams, m->part.p);
+    const int nwb = (FI_NB + 63) / 64;
+    k_mlp_sum<<<nwb + (int)((m->nparams + 1023) / 1024), 1024, 0, s>>>(m->nparams, S, m->part.p, nb, m->tbias.p,
+                                                                      m->dboff.p, nwb, m->grads.p);
+    HIPCHK(hipGetLastError());
+    return FIPC_OK;
+}
+
 // gradient of the mean squared error over n rows (X, T on the device) into
-// m->grads; the loss partials are left in m->loss (nblk(n n_out) floats)
+// m->grads; the loss partials are left in m->loss (mlp_loss_parts floats)
 static int mlp_backward(fipc_mlp* m, hipStream_t s, int n, const float* X, const float* T)
 {
+    if (m->fused) return mlp_backward_fused(m, s, n, X, T);
     STCHK(mlp_forward(m, s, n, X, true));
     long ny = (long)n * m->n_out;
     float* dZ = m->dA.p;   // gradient at the current layer's pre-activation
     float* dH = m->dB.p;
     k_mse<<<nblk(ny), TPB, 0, s>>>(ny, 1.f / (float)ny, m->H[m->L].p, T, dZ, m->loss.p);
     HIPCHK(hipGetLastError());
-    // split-K partials of dW: slices of at most 1024 rows
+    // split-K partials of dW and of the bias gradients: slices of at most 1024 rows
     int S = std::max(1, std::min(32, (n + 1023) / 1024));
     for (int l = m->L - 1; l >= 0; l--) {
         int fi = m->dim[l], fo = m->dim[l + 1];
@@ -460,7 +824,8 @@ static int mlp_backward(fipc_mlp* m, hipStream_t s, int n, const float* X, const
         STCHK(gemm(s, fi, fo, n, Hin, 1, fi, dZ, fo, 1, m->part.p, fo, EPI_NONE, nullptr, nullptr, nullptr, S,
                    (long)fi * fo));
         k_sum_slices<<<nblk((long)fi * fo), TPB, 0, s>>>((long)fi * fo, S, m->part.p, m->grads.p + m->woff[l]);
-        k_colsum<<<(fo + 63) / 64, 256, 0, s>>>(n, fo, dZ, m->grads.p + m->boff[l]);
+        k_colsum<<<dim3((fo + 63) / 64, S), 256, 0, s>>>(n, fo, (n + S - 1) / S, dZ, m->part.p);
+        k_sum_slices<<<nblk(fo), TPB, 0, s>>>(fo, S, m->part.p, m->grads.p + m->boff[l]);
         HIPCHK(hipGetLastError());
         if (l > 0) {
             // dZ_{l} = (dZ W_l^T) * silu'(Z_l)
@@ -481,15 +846,9 @@ int mlp_dims(const fipc_mlp* m, int* n_in, int* n_out)
 static int mlp_pack(fipc_mlp* m, hipStream_t s)
 {
     if (m->wt_ok) return FIPC_OK;
-    long total = 0;
-    for (int l = 0; l < m->L; l++) total += (long)(l == m->L - 1 ? 32 : m->dim[l + 1]) * m->dim[l];
+    const long total = FI_WT + FI_WN;
     STCHK(ensure(m->wt, total));
-    long o = 0;
-    for (int l = 0; l < m->L; l++) {
-        int fi = m->dim[l], fo = m->dim[l + 1], rows = l == m->L - 1 ? 32 : fo;
-        k_pack_wt<<<nblk((long)rows * fi), TPB, 0, s>>>(fi, fo, rows, m->params.p + m->woff[l], m->wt.p + o);
-        o += (long)rows * fi;
-    }
+    k_pack_weights<<<nblk(total), TPB, 0, s>>>(m->params.p, m->dboff.p, m->wt.p, total);
     HIPCHK(hipGetLastError());
     m->wt_ok = true;
     return FIPC_OK;
@@ -602,6 +961,7 @@ extern "C" int fipc_mlp_destroy(fipc_mlp* m)
     for (auto& v : m->Z) release(v);
     release(m->X); release(m->T); release(m->dA); release(m->dB); release(m->part); release(m->loss);
     release(m->dsX); release(m->dsT); release(m->wt); release(m->dboff);
+    release(m->tA); release(m->tG); release(m->tbias);
     if (m->s) (void)hipStreamDestroy(m->s);
     delete m;
     return FIPC_OK;
@@ -652,7 +1012,7 @@ extern "C" int fipc_mlp_grad(fipc_mlp* m, int n, const float* X, const float* T,
     HIPCHK(hipMemcpyAsync(m->X.p, X, (size_t)n * m->n_in * 4, hipMemcpyHostToDevice, m->s));
     HIPCHK(hipMemcpyAsync(m->T.p, T, (size_t)n * m->n_out * 4, hipMemcpyHostToDevice, m->s));
     STCHK(mlp_backward(m, m->s, n, m->X.p, m->T.p));
-    int nb = nblk((long)n * m->n_out);
+    int nb = mlp_loss_parts(m, n);
     std::vector<float> lp(nb);
     HIPCHK(hipMemcpyAsync(lp.data(), m->loss.p, nb * 4, hipMemcpyDeviceToHost, m->s));
     if (grad) HIPCHK(hipMemcpyAsync(grad, m->grads.p, m->nparams * 4, hipMemcpyDeviceToHost, m->s));
@@ -706,7 +1066,7 @@ extern "C" int fipc_mlp_train(fipc_mlp* m, int iters, int batch, float lr, unsig
 {
     if (!m || iters < 0 || batch <= 0 || m->ds_n == 0) return FIPC_ERR_ARG;
     STCHK(mlp_reserve(m, batch, true));
-    int nb = nblk((long)batch * m->n_out);
+    int nb = mlp_loss_parts(m, batch);
     DVec<float> lossall;
     STCHK(ensure(lossall, (size_t)iters * nb + 1));
     const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;

@@ -125,3 +125,48 @@ def test_grid_queries_visit_every_pair_once(n, copies, spread):
     sim.find_constraints()
     assert tuple(sim.search_counts()) == _brute_pairs(moved, sc, sc.dhat)
     sim.close()
+
+
+@pytest.mark.parametrize("rows", [1, 31, 32, 33, 63, 64, 65, 511, 512, 513, 1100])
+def test_network_gradient_over_row_remainders(rows):
+    """Loss and gradient of the warm-start shape at the edges of its 32-row blocks
+    and row slices, against the same network in float64 with inputs of every
+    product rounded to BF16 (8 bits): each rounding moves a product by at most
+    2^-9 of its size, and 10 of them follow one another."""
+    from fastipc_amd.warmstart import WarmStartMLP
+    rng = np.random.default_rng(rows)
+    net = WarmStartMLP(seed=rows)
+    X = rng.standard_normal((rows, 16)).astype(np.float32)
+    T = rng.standard_normal((rows, 3)).astype(np.float32)
+    loss, grad = net.grad(X, T)
+    w = net.params().astype(np.float64)
+
+    def bf(a):
+        u = np.ascontiguousarray(a, np.float32).view(np.uint32).astype(np.uint64)
+        return ((((u + 0x7FFF + ((u >> 16) & 1)) >> 16) << 16).astype(np.uint32)).view(np.float32).astype(np.float64)
+
+    dims, o, Ws, bs = [16, 256, 256, 256, 256, 3], 0, [], []
+    for a, b in zip(dims, dims[1:]):
+        Ws.append(w[o:o + a * b].reshape(a, b))
+        bs.append(w[o + a * b:o + a * b + b])
+        o += a * b + b
+    A, Z, h = [], [], X.astype(np.float64)
+    for k, (W, b) in enumerate(zip(Ws, bs)):
+        A.append(bf(h))
+        z = A[-1] @ bf(W) + b
+        Z.append(z)
+        h = z / (1 + np.exp(-z)) if k < 4 else z
+    d = h - T
+    assert abs(loss - (d ** 2).mean()) <= 1e-3 * (d ** 2).mean()
+    G, want = 2 * d / d.size, [None] * 5
+    for k in range(4, -1, -1):
+        want[k] = np.concatenate([(A[k].T @ bf(G)).ravel(), G.sum(0)])
+        if k:
+            s = 1 / (1 + np.exp(-Z[k - 1]))
+            G = (bf(G) @ bf(Ws[k]).T) * (s * (1 + Z[k - 1] * (1 - s)))
+    o = 0
+    for g in want:
+        got = grad[o:o + g.size]
+        assert np.linalg.norm(got - g) <= 10 * 2.0 ** -9 * np.linalg.norm(g), np.linalg.norm(got - g) / np.linalg.norm(g)
+        o += g.size
+    net.close()
