@@ -416,7 +416,7 @@ __global__ void k_pack_weights(const float* __restrict__ params, const long* __r
 //  - k_mlp_sum: the slices' and the blocks' sums.
 // Layer by layer, with FP32 activations in HBM and a column sum of 8,192 rows
 // in four workgroups (385 us a layer), loss and gradient of 8,192 rows took
-// 3.0 ms of kernels; like this 168 us.
+// 3.0 ms of kernels; like this 85 us.
 // ---------------------------------------------------------------------------
 struct TrainBufs {
     __bf16* A;      // A_0 [16][ld], then A_1 .. A_4 [256][ld]
@@ -490,24 +490,29 @@ __device__ __forceinline__ void ft_store(const float (&v)[2][16], __bf16 (*H)[FI
 }
 // column sums over the block's 32 rows: each step hands half of the values to the
 // lane across, so 31 exchanges reduce 32 values; lane l % 32 ends with value l % 32
+template <int N>
+__device__ __forceinline__ float ft_fold(const float (&w)[2 * N], int lane)
+{
+    float h[N];
+    const bool up = lane & N;
+#pragma unroll
+    for (int k = 0; k < N; k++) {
+        const float lo = w[k], hi = w[k + N];
+        h[k] = (up ? hi : lo) + __shfl_xor(up ? lo : hi, N, 64);
+    }
+    if constexpr (N == 1) return h[0];
+    else return ft_fold<N / 2>(h, lane);
+}
 __device__ __forceinline__ void ft_colsum(const float (&v)[2][16], float* __restrict__ out, int f0, int lane)
 {
     float w[32];
 #pragma unroll
     for (int k = 0; k < 32; k++) w[k] = v[k >> 4][k & 15];
-#pragma unroll
-    for (int s = 16, n = 16; s > 0; s >>= 1, n >>= 1) {
-        const bool up = lane & s;
-#pragma unroll
-        for (int k = 0; k < n; k++) {
-            const float send = up ? w[k] : w[k + n], keep = up ? w[k + n] : w[k];
-            w[k] = keep + __shfl_xor(send, s, 64);
-        }
-    }
+    const float sum = ft_fold<16>(w, lane);
     const int k = lane & 31, j = k & 15;
-    out[f0 + 32 * (k >> 4) + 8 * (j >> 2) + 4 * (lane >> 5) + (j & 3)] = w[0];
+    out[f0 + 32 * (k >> 4) + 8 * (j >> 2) + 4 * (lane >> 5) + (j & 3)] = sum;
 }
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2)))
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1)))
 k_mlp_fwdbwd(int n, const float* __restrict__ X, const float* __restrict__ T, const __bf16* __restrict__ Wt,
              const float* __restrict__ params, const long* __restrict__ boff, float inv, TrainBufs tb)
 {
