@@ -3,12 +3,9 @@
 #include <mutex>
 #include "fipc_ctx.h"
 
-#define TPB 256
-static inline int nblk(long n, int t = TPB) { return (int)((n + t - 1) / t); }
-
-// the batched CCD kernel of fipc_broad.hip (one thread per pair)
-__global__ void k_batch_ccd(int type, int n, const double* pts, const double* disp, double eta, const double* d2,
-                            double* toc);
+// the batched CCD of fipc_broad.hip on device arrays
+int fipc_launch_batch_ccd(int type, int n, const double* pts, const double* disp, double eta, const double* d2,
+                          double* toc);
 
 // ---- the same batch without device allocation -------------------------------
 // For callers that cannot call hipMalloc (graph capture, serving loops): the
@@ -51,8 +48,7 @@ extern "C" int fipc_batch_ccd_noalloc(int type, int n, const double* pts, const 
     HIPCHK(hipMemcpy(dp, pts, (size_t)n * 96, hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(dd, disp, (size_t)n * 96, hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(d2, dist2, (size_t)n * 8, hipMemcpyHostToDevice));
-    k_batch_ccd<<<nblk(n), TPB>>>(type, n, dp, dd, eta, d2, dt);
-    HIPCHK(hipGetLastError());
+    STCHK(fipc_launch_batch_ccd(type, n, dp, dd, eta, d2, dt));
     HIPCHK(hipMemcpy(toc, dt, (size_t)n * 8, hipMemcpyDeviceToHost));
     return FIPC_OK;
 }

@@ -170,3 +170,20 @@ def test_network_gradient_over_row_remainders(rows):
         assert np.linalg.norm(got - g) <= 10 * 2.0 ** -9 * np.linalg.norm(g), np.linalg.norm(got - g) / np.linalg.norm(g)
         o += g.size
     net.close()
+
+
+@pytest.mark.parametrize("kind", [0, 1])
+def test_batch_ccd_does_not_depend_on_the_number_of_pairs(kind):
+    """A pair's time is the same bits alone and in full and partial blocks of 64."""
+    rng = np.random.default_rng(kind)
+    P = rng.uniform(-1, 1, (200, 12))
+    D = rng.normal(0, 1, (200, 12))
+    d2 = np.full(200, 1e-4)
+    toc = np.zeros(200)
+    _lib.call("fipc_batch_ccd", kind, 200, _lib.dptr(P), _lib.dptr(D), 0.2, _lib.dptr(d2), _lib.dptr(toc))
+    assert ((toc >= 0) & (toc <= 1)).all() and (toc < 1).any() and (toc == 1).any()
+    for n in (1, 63, 64, 65, 128, 129):
+        t = np.zeros(n)
+        _lib.call("fipc_batch_ccd", kind, n, _lib.dptr(P[:n].copy()), _lib.dptr(D[:n].copy()), 0.2,
+                  _lib.dptr(d2[:n].copy()), _lib.dptr(t))
+        assert np.array_equal(t, toc[:n]), n
