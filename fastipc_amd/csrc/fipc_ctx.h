@@ -143,6 +143,7 @@ struct fipc_ctx {
     int count[NTYPES] = {0};
     int raw_count[NTYPES] = {0};
     DVec<int> rows[NTYPES];
+    DVec<int> rows_small[NTYPES];  // sorted rows of a small set, swapped with rows[t]
     DVec<int> rows_tmp;    // the sort of the four-index types writes here, then swaps
     DVec<double> cH[NTYPES];  // the rows' unprojected Hessians, between the assembly's two contact launches
     // Contact vertices: every (row, vertex) slot of the seven types, slot

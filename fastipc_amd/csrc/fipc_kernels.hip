@@ -1640,7 +1640,7 @@ extern "C" int fipc_destroy(fipc_ctx* c)
     release(c->vcent);
     release(c->tile_meta); release(c->tile_tcode); release(c->tile_vcode); release(c->tile_ppos); release(c->tile_vpos);
     release(c->tile_pptr); release(c->tile_vptr); release(c->tile_bpart); release(c->tile_gpart);
-    for (int t = 0; t < NTYPES; t++) { release(c->rows[t]); release(c->cH[t]); }
+    for (int t = 0; t < NTYPES; t++) { release(c->rows[t]); release(c->rows_small[t]); release(c->cH[t]); }
     release(c->cv_keys); release(c->cv_vals); release(c->cv_keys2); release(c->cv_slot); release(c->cv_head);
     release(c->cv_vert); release(c->cv_ptr); release(c->cv_count); release(c->cgrad);
     release(c->cv_place); release(c->cv_ids); release(c->cv_meta); release(c->cv_H); release(c->cv_Hf);

@@ -187,3 +187,41 @@ def test_batch_ccd_does_not_depend_on_the_number_of_pairs(kind):
         _lib.call("fipc_batch_ccd", kind, n, _lib.dptr(P[:n].copy()), _lib.dptr(D[:n].copy()), 0.2,
                   _lib.dptr(d2[:n].copy()), _lib.dptr(t))
         assert np.array_equal(t, toc[:n]), n
+
+
+@pytest.mark.parametrize("n,m,layers", [(3, 1, 2), (6, 2, 2), (9, 2, 2), (12, 2, 2), (12, 2, 3)])
+def test_row_sets_on_both_sides_of_the_one_launch_sort(n, m, layers):
+    """Constraint rows, in np.unique order, against the oracle's search: sets below
+    and above 1,024 rows, after one another on one context."""
+    from fastipc_amd import scene as S
+    from fastipc_amd.newton import NewtonIPC
+    from oracle.newton import OracleIPC
+    xc, tc = S.lattice(n)
+    edge = (n - 1) * S.LATTICE_SPACING
+    xs, ts, nv = [], [], 0
+    for layer in range(layers):
+        for i in range(m):
+            for k in range(m):
+                xs.append(xc + [(1.06 * i + 0.31 * (layer % 2)) * edge, layer * (edge + 1e-3) + 1e-3,
+                                (1.06 * k + 0.17 * (layer % 2)) * edge])
+                ts.append(tc + nv)
+                nv += len(xc)
+    gx, gt = S.box([-edge, -0.1, -edge], [(m + 2) * edge, 0.0, (m + 2) * edge])
+    x, tets = np.concatenate(xs + [gx]), np.concatenate(ts + [gt + nv]).astype(np.int32)
+    one = np.ones(len(tets))
+    sc = S.Scene(name="pile", x=x, tets=tets, density=1000 * one, youngs=1e5 * one, poisson=0.4 * one,
+                 dirichlet_mask=np.arange(len(x)) >= nv, dt=0.01)
+    sim, orc = NewtonIPC(sc), OracleIPC(sc)
+    rng = np.random.default_rng(n)
+    for lift in (0.0, 2.0, 0.0):  # all in contact, the bodies apart, in contact again
+        state = sc.x.copy()
+        state[:nv] += rng.uniform(-1e-4, 1e-4, (nv, 3))
+        state[:nv, 1] += lift * edge * (sc.x[:nv, 1] > 0.5 * edge)
+        sim.set_state(state, np.zeros_like(state))
+        sim.find_constraints()
+        orc.x = np.ascontiguousarray(state)
+        orc.find_constraints()
+        got = sim.constraints(sort=False)
+        for k, rows in orc.constraints().items():
+            assert np.array_equal(got[k], rows), (k, len(got[k]), len(rows))
+    sim.close()
