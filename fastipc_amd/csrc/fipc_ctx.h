@@ -126,14 +126,14 @@ struct fipc_ctx {
     DVec<int> cpos, bcptr, vcptr, vcent;
     DVec<int> gorder;      // the gather's block order: diagonal blocks first
     // FP32 mode's tiled pass (k_elastic_tile): nchunk chunks of consecutive
-    // tets, TILE_META int4 each; per (slot, tet) and (corner, tet) the LDS
+    // tets, TILE_META int4 each; per tet, for its slots and corners, the LDS
     // index | colour << 8 of the entry it adds to; per (chunk, block) and
     // (chunk, vertex) the position of the partial record, whose runs per
     // block / vertex are tile_pptr / tile_vptr
     int nchunk = 0;
     long tile_nbpart = 0, tile_nvpart = 0;
     DVec<int4> tile_meta;
-    DVec<unsigned short> tile_tcode, tile_vcode;
+    DVec<unsigned short> tile_code;  // 16 per tet: its ten block slots, its corners, two unused
     DVec<int> tile_ppos, tile_vpos, tile_pptr, tile_vptr;
     DVec<float> tile_bpart;
     DVec<double> tile_gpart;

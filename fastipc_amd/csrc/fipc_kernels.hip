@@ -260,14 +260,15 @@ __device__ __forceinline__ void tile_add(A* lds, unsigned code, int ncol, const 
 }
 
 __global__ void __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(3)))
-k_elastic_tile(int nchunk, int nt, const int4* __restrict__ meta, const unsigned short* __restrict__ tcode,
-               const unsigned short* __restrict__ vcode, const int* __restrict__ ppos, const int* __restrict__ vpos,
+k_elastic_tile(int nchunk, const int4* __restrict__ meta, const uint4* __restrict__ code,
+               const int* __restrict__ ppos, const int* __restrict__ vpos,
                const int* __restrict__ tets, const double* __restrict__ IB, const double* __restrict__ vol,
                const double* __restrict__ la, const double* __restrict__ mu, const double* __restrict__ x,
                double dt2, float* __restrict__ bpart, double* __restrict__ gpart)
 {
     __shared__ float lb[TPB / 64][TILE_MAXB * 9];
     __shared__ double lg[TPB / 64][TILE_MAXV * 3];
+    __shared__ int lp[TPB / 64][TILE_MAXB];  // the block records' places
     const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane((int)blockIdx.x * (TPB / 64) + wv);
     if (w >= nchunk) return;
@@ -280,11 +281,22 @@ k_elastic_tile(int nchunk, int nt, const int4* __restrict__ meta, const unsigned
                             (unsigned)__builtin_amdgcn_readfirstlane(m2.z), (unsigned)__builtin_amdgcn_readfirstlane(m2.w)};
     float* B = lb[wv];
     double* G = lg[wv];
-    for (int i = lane; i < 9 * nb; i += 64) B[i] = 0.0f;
-    for (int i = lane; i < 3 * nvx; i += 64) G[i] = 0.0;
-    wave_step();
+    // everything the tail and the sums need of the tables is loaded here, ahead
+    // of the arithmetic that hides it: the records' places (to LDS) and the tet's
+    // 14 codes.  Loaded where they are used, behind the fences of the sums and one
+    // by one in the tail's loop, the pass took 278 us on 948,405 tets, like this 218
     const bool act = lane < n;
     const int e = act ? e0 + lane : e0;  // idle lanes recompute the first tet and add nothing
+    const uint4 c0 = code[2 * (size_t)e], c1 = code[2 * (size_t)e + 1];
+    const unsigned cd[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
+    int pp[TILE_MAXB / 64];
+#pragma unroll
+    for (int k = 0; k < TILE_MAXB / 64; k++) pp[k] = lane + 64 * k < nb ? ppos[pbase + lane + 64 * k] : 0;
+    for (int i = lane; i < 9 * nb; i += 64) B[i] = 0.0f;
+    for (int i = lane; i < 3 * nvx; i += 64) G[i] = 0.0;
+#pragma unroll
+    for (int k = 0; k < TILE_MAXB / 64; k++) lp[wv][lane + 64 * k] = pp[k];
+    wave_step();
     int t[4];
     double F[9], Bm[4][3];
     tet_load(tets, IB, x, e, t, F, Bm);
@@ -298,7 +310,7 @@ k_elastic_tile(int nchunk, int nt, const int4* __restrict__ meta, const unsigned
 #pragma unroll
         for (int i = 0; i < 3; i++) g[i] = (P[i * 3] * Bm[a][0] + P[i * 3 + 1] * Bm[a][1] + P[i * 3 + 2] * Bm[a][2]) * sc;
         const int k = 10 + a;
-        tile_add<3, double>(G, vcode[(size_t)a * nt + e], (int)((cw[k >> 2] >> (8 * (k & 3))) & 0xffu), g, act);
+        tile_add<3, double>(G, (cd[k >> 1] >> (16 * (k & 1))) & 0xffffu, (int)((cw[k >> 2] >> (8 * (k & 3))) & 0xffu), g, act);
     }
     NHFactor f;
     nh_factor(F, lae, mue, f);
@@ -314,10 +326,11 @@ k_elastic_tile(int nchunk, int nt, const int4* __restrict__ meta, const unsigned
 #pragma unroll
                 for (int j = 0; j < 3; j++) o[i * 3 + j] = blk[j * 3 + i];
         }
-        tile_add<9, float>(B, tcode[(size_t)k * nt + e], (int)((cw[k >> 2] >> (8 * (k & 3))) & 0xffu), o, act);
+        tile_add<9, float>(B, (cd[k >> 1] >> (16 * (k & 1))) & 0xffffu, (int)((cw[k >> 2] >> (8 * (k & 3))) & 0xffu), o, act);
     });
     // nine (three) consecutive lanes write a record's consecutive entries
-    for (int i = lane; i < 9 * nb; i += 64) bpart[(size_t)ppos[pbase + i / 9] * 9 + i % 9] = B[i];
+#pragma unroll 4
+    for (int i = lane; i < 9 * nb; i += 64) bpart[(size_t)lp[wv][i / 9] * 9 + i % 9] = B[i];
     for (int i = lane; i < 3 * nvx; i += 64) gpart[(size_t)vpos[vbase + i / 3] * 3 + i % 3] = G[i];
 }
 
@@ -1638,7 +1651,7 @@ extern "C" int fipc_destroy(fipc_ctx* c)
     release(c->brow); release(c->tetH); release(c->tetg); release(c->bcptr); release(c->gorder); release(c->cpos); release(c->vcptr);
     release(c->lptr); release(c->lent);
     release(c->vcent);
-    release(c->tile_meta); release(c->tile_tcode); release(c->tile_vcode); release(c->tile_ppos); release(c->tile_vpos);
+    release(c->tile_meta); release(c->tile_code); release(c->tile_ppos); release(c->tile_vpos);
     release(c->tile_pptr); release(c->tile_vptr); release(c->tile_bpart); release(c->tile_gpart);
     for (int t = 0; t < NTYPES; t++) { release(c->rows[t]); release(c->rows_small[t]); release(c->cH[t]); }
     release(c->cv_keys); release(c->cv_vals); release(c->cv_keys2); release(c->cv_slot); release(c->cv_head);
@@ -1676,7 +1689,7 @@ extern "C" int fipc_destroy(fipc_ctx* c)
 static int build_tiles(fipc_ctx* c, int nv, int nt, int nnzb, const int* tets, const std::vector<int>& cblock)
 {
     std::vector<int4> meta;
-    std::vector<unsigned short> tcode((size_t)std::max(nt, 1) * 10), vcode((size_t)std::max(nt, 1) * 4);
+    std::vector<unsigned short> code((size_t)std::max(nt, 1) * 16, 0);
     std::vector<int> cblk, cvert;  // per (chunk, local index): the block / vertex
     std::vector<int> bstamp(std::max(nnzb, 1), -1), blid(std::max(nnzb, 1)), vstamp(nv, -1), vlid(nv);
     std::vector<int> ccnt(14 * (size_t)TILE_MAXB);
@@ -1696,14 +1709,14 @@ static int build_tiles(fipc_ctx* c, int nv, int nt, int nnzb, const int* tets, c
                 int b = cblock[(size_t)e * 10 + k];
                 if (bstamp[b] != ch) { bstamp[b] = ch; blid[b] = nb++; cblk.push_back(b); }
                 int col = ccnt[(size_t)k * TILE_MAXB + blid[b]]++;
-                tcode[(size_t)k * nt + e] = (unsigned short)(blid[b] | col << 8);
+                code[(size_t)e * 16 + k] = (unsigned short)(blid[b] | col << 8);
                 ncol[k] = (unsigned char)std::max<int>(ncol[k], col + 1);
             }
             for (int a = 0; a < 4; a++) {
                 int v = tets[4 * e + a];
                 if (vstamp[v] != ch) { vstamp[v] = ch; vlid[v] = nvx++; cvert.push_back(v); }
                 int col = ccnt[(size_t)(10 + a) * TILE_MAXB + vlid[v]]++;
-                vcode[(size_t)a * nt + e] = (unsigned short)(vlid[v] | col << 8);
+                code[(size_t)e * 16 + 10 + a] = (unsigned short)(vlid[v] | col << 8);
                 ncol[10 + a] = (unsigned char)std::max<int>(ncol[10 + a], col + 1);
             }
             e++;
@@ -1730,8 +1743,7 @@ static int build_tiles(fipc_ctx* c, int nv, int nt, int nnzb, const int* tets, c
     c->nchunk = ch;
     if (meta.empty()) meta.push_back(make_int4(0, 0, 0, 0));
     STCHK(upload(c->tile_meta, meta.data(), meta.size(), c->s));
-    STCHK(upload(c->tile_tcode, tcode.data(), tcode.size(), c->s));
-    STCHK(upload(c->tile_vcode, vcode.data(), vcode.size(), c->s));
+    STCHK(upload(c->tile_code, code.data(), code.size(), c->s));
     STCHK(upload(c->tile_ppos, ppos.data(), ppos.size(), c->s));
     STCHK(upload(c->tile_vpos, vpos.data(), vpos.size(), c->s));
     STCHK(upload(c->tile_pptr, pptr.data(), pptr.size(), c->s));
@@ -2187,7 +2199,7 @@ extern "C" int fipc_assemble(fipc_ctx* c, int precision)
     if (c->nt) {
         if (precision == 1)
             k_elastic_tile<<<(c->nchunk + TPB / 64 - 1) / (TPB / 64), TPB, 0, c->s>>>(
-                c->nchunk, c->nt, c->tile_meta.p, c->tile_tcode.p, c->tile_vcode.p, c->tile_ppos.p, c->tile_vpos.p,
+                c->nchunk, c->tile_meta.p, (const uint4*)c->tile_code.p, c->tile_ppos.p, c->tile_vpos.p,
                 c->tets.p, c->IB.p, c->vol.p, c->la.p, c->mu.p, c->x.p, c->dt * c->dt, c->tile_bpart.p,
                 c->tile_gpart.p);
         else
