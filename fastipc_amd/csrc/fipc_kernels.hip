@@ -977,6 +977,8 @@ struct ContactSet {
 // table but ptr: through slot numbers, row tables and per-type Hessians, a chain
 // of five dependent loads, a product on two cubes in contact (520 rows) took
 // 13.7 us against 9.2, and on 27 cubes of 16^3 (29,367 rows) 40.3 against 32.1.
+// All of a slot's loads are issued before its sums: one latency for the slot, not
+// one for each of its points (27 cubes 31.1 -> 27.2 us).
 template <class V>
 __device__ __forceinline__ void contact_vertex_spmv(const ContactSet& cs, const V* __restrict__ p, int e, int e1,
                                                     double* s)
@@ -991,26 +993,28 @@ __device__ __forceinline__ void contact_vertex_spmv(const ContactSet& cs, const 
         if (e + CV_G < e1) { nid = cs.sd.ids[e + CV_G]; nmt = cs.sd.meta[e + CV_G]; }
         const bool f32 = cs.sd.Hf && !(mt & SLOT_KEEP64);
         const int w[4] = {id.x, id.y, id.z, id.w};
+        double h[4][9], q[4][3];
+#pragma unroll
+        for (int b = 0; b < 4; b++)
+            if (b < K) {
+#pragma unroll
+                for (int d = 0; d < 3; d++) q[b][d] = (double)p[3 * w[b] + d];
+                if (f32) {
+#pragma unroll
+                    for (int k = 0; k < 9; k++) h[b][k] = (double)cs.sd.Hf[36 * (size_t)e + 9 * b + k];
+                } else {
+#pragma unroll
+                    for (int k = 0; k < 9; k++) h[b][k] = cs.sd.H[36 * (size_t)e + 9 * b + k];
+                }
+            }
         double a0 = 0.0, a1 = 0.0, a2 = 0.0;
 #pragma unroll
-        for (int b = 0; b < 4; b++) {
+        for (int b = 0; b < 4; b++)
             if (b < K) {
-                const double p0 = (double)p[3 * w[b]], p1 = (double)p[3 * w[b] + 1], p2 = (double)p[3 * w[b] + 2];
-                double h[9];
-                if (f32) {
-                    const float* q = cs.sd.Hf + 36 * (size_t)e + 9 * b;
-#pragma unroll
-                    for (int k = 0; k < 9; k++) h[k] = (double)q[k];
-                } else {
-                    const double* q = cs.sd.H + 36 * (size_t)e + 9 * b;
-#pragma unroll
-                    for (int k = 0; k < 9; k++) h[k] = q[k];
-                }
-                a0 += h[0] * p0 + h[1] * p1 + h[2] * p2;
-                a1 += h[3] * p0 + h[4] * p1 + h[5] * p2;
-                a2 += h[6] * p0 + h[7] * p1 + h[8] * p2;
+                a0 += h[b][0] * q[b][0] + h[b][1] * q[b][1] + h[b][2] * q[b][2];
+                a1 += h[b][3] * q[b][0] + h[b][4] * q[b][1] + h[b][5] * q[b][2];
+                a2 += h[b][6] * q[b][0] + h[b][7] * q[b][1] + h[b][8] * q[b][2];
             }
-        }
         s[0] += a0; s[1] += a1; s[2] += a2;
     }
 }
@@ -1018,8 +1022,12 @@ __device__ __forceinline__ void contact_vertex_spmv(const ContactSet& cs, const 
 // places (an upper bound from the number of slots, which fixes the order of the
 // sum), the BSR blocks' those after; the places of the contact blocks that are
 // not launched, or have no vertices, are not read.
+//
+// Four waves on a SIMD, stated: a slot's 48 values in flight take 129 registers,
+// one over what lets four run, and the BSR part of a large mesh needs them (1M
+// tets in FP32: 33.9 us at three waves, 24.8 at four, 27.0 with spills at five).
 template <class T, class V>
-__global__ void __launch_bounds__(TPB)
+__global__ void __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(4)))
 k_spmv(int nv, const int* __restrict__ rowptr, const int* __restrict__ col, const int* __restrict__ lptr,
        const int2* __restrict__ lent, const T* __restrict__ val, const V* __restrict__ p, V* __restrict__ q,
        double* qc, const unsigned char* __restrict__ dmask, ContactSet cs, int nl_c, int nb_c, int nb_bsr,
