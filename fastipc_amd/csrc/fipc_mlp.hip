@@ -237,7 +237,7 @@ constexpr int FI_THREADS = 4 * (FI_ROWS / FI_WROWS) * 64;
 // D[feature][row] += W[feature][k..k+15] . H[row][k..k+15] over the layer's
 // fan-in KIN for NF 32-feature tiles from f0 and RT 32-row tiles from rbase.
 // The A operand is a weight fragment (8 consecutive k of one output feature,
-// one 16-byte load from the transposed BF16 weights), the B operand an
+// one 16-byte load from the packed BF16 weights), the B operand an
 // activation fragment (8 consecutive k of one row, one 16-byte LDS read);
 // the next k step's weight fragments are loaded before this step's products.
 template <int NF, int RT>
@@ -262,7 +262,7 @@ __device__ __forceinline__ void fi_layer(const __bf16* __restrict__ W, const __b
     bf16x8 a[NF], an[NF];
 #pragma unroll
     for (int f = 0; f < NF; f++) {
-        wp[f] = W + (long)(f0 + f * 32 + (lane & 31)) * KIN + (lane >> 5) * 8;
+        wp[f] = W + (long)(f0 / 32 + f) * 32 * KIN + lane * 8;
         a[f] = *(const bf16x8*)wp[f];
     }
     if (KIN == 16) {
@@ -274,11 +274,11 @@ __device__ __forceinline__ void fi_layer(const __bf16* __restrict__ W, const __b
     // reloads its own last step rather than read past the row)
     for (int k0 = 0; k0 < KIN; k0 += 32) {
 #pragma unroll
-        for (int f = 0; f < NF; f++) an[f] = *(const bf16x8*)(wp[f] + k0 + 16);
+        for (int f = 0; f < NF; f++) an[f] = *(const bf16x8*)(wp[f] + 32 * (k0 + 16));
         fi_step<NF, RT>(a, H, rbase, lane, k0, acc);
         const int kn = k0 + 32 < KIN ? k0 + 32 : KIN - 16;
 #pragma unroll
-        for (int f = 0; f < NF; f++) a[f] = *(const bf16x8*)(wp[f] + kn);
+        for (int f = 0; f < NF; f++) a[f] = *(const bf16x8*)(wp[f] + 32 * kn);
         fi_step<NF, RT>(an, H, rbase, lane, k0 + 16, acc);
     }
 }
@@ -315,16 +315,16 @@ __device__ __forceinline__ void fi_silu_store(const floatx16 (&acc)[2][RT], cons
 // Fused inference for the warm-start shape (16 -> 4 x 256 SiLU -> 3): a block
 // takes FI_ROWS rows through all five layers; the activations stay in LDS as
 // BF16 (the products' input precision) and never touch HBM.  Weights are read
-// from L2 as BF16 transposed per layer, Wt[n][k] (the last layer padded to 32
-// rows of zeros).  In the hidden layers wave w owns output features
+// from L2 as BF16 fragments per layer (k_pack_weights; the last layer padded to
+// 32 rows of zeros).  In the hidden layers wave w owns output features
 // 64 (w % 4) .. +64 (two 32-feature MFMA tiles) of its FI_RT 32-row tiles:
 // each weight fragment feeds FI_RT MFMAs, each activation fragment two.  The
 // output layer's 32-row tiles are shared out over all the block's waves.
 // The weight fragments come from L1/L2, so rows per wave set the loads per
 // product: 200k rows take 199 us with 2 row tiles (108 VGPRs, 4 waves per
 // SIMD), 159 us with 3, 151 us with 4 (192 VGPRs, 2 waves per SIMD, two
-// 128-row blocks per CU), all with the same bits; 5 or more row tiles fit only
-// one wave per SIMD.  The accumulation order over k is the generic GEMM's.
+// 128-row blocks per CU), all with the same bits and with weights row by row (132
+// us as fragments); 5 or more row tiles fit only one wave per SIMD.  The accumulation order over k is the generic GEMM's.
 // ---------------------------------------------------------------------------
 __global__ void __launch_bounds__(FI_THREADS) __attribute__((amdgpu_waves_per_eu(FI_RT <= 2 ? 4 : 2)))
 k_mlp_infer(int n, const float* __restrict__ X, const __bf16* __restrict__ Wt, const float* __restrict__ params,
@@ -373,10 +373,22 @@ k_mlp_infer(int n, const float* __restrict__ X, const __bf16* __restrict__ Wt, c
 }
 // BF16 weights of the warm-start shape from the FP32 parameters, one launch: per
 // layer Wt[n][k] (transposed, the last padded to 32 rows), then, for the
-// backward products, W[k][n] of layers 1 to 4 (the last padded to 16 columns)
+// backward products, W[k][n] of layers 1 to 4 (the last padded to 16 columns).
+// Each matrix is stored as its A fragments: 32 rows by 16 columns, 8 consecutive
+// columns per lane, lane after lane, so a wave's load is 1 KB in a row.  Row by
+// row, a load touched 32 bytes of each of 32 lines, and the lines of two blocks
+// did not stay in L1 until their next quarter was read: inference of 200k rows
+// 151 us row by row, 132 in fragments.
 constexpr int FI_L = 5, FI_IN = 16, FI_OUT = 3;
 constexpr long FI_WT = (long)FI_W * FI_IN + 3L * FI_W * FI_W + 32L * FI_W;  // elements of the first part
 constexpr long FI_WN = 3L * FI_W * FI_W + 16L * FI_W;                       // and of the second
+// row and column of the j-th element of a matrix of ld columns in fragment order
+__device__ __forceinline__ void fi_frag(int j, int ld, int& row, int& col)
+{
+    const int lane = (j >> 3) & 63, t = j >> 9, steps = ld / 16;
+    row = t / steps * 32 + (lane & 31);
+    col = t % steps * 16 + (lane >> 5) * 8 + (j & 7);
+}
 __global__ void k_pack_weights(const float* __restrict__ params, const long* __restrict__ boff, __bf16* __restrict__ w,
                                long total)
 {
@@ -389,14 +401,16 @@ __global__ void k_pack_weights(const float* __restrict__ params, const long* __r
         long size = (long)FI_W * FI_IN;
         while (j >= size) { j -= size; l++; size = l == FI_L - 1 ? 32L * FI_W : (long)FI_W * FI_W; }
         const int fi = l == 0 ? FI_IN : FI_W, fo = l == FI_L - 1 ? FI_OUT : FI_W;
-        const int n = (int)(j / fi), k = (int)(j % fi);
+        int n, k;
+        fi_frag((int)j, fi, n, k);
         if (n < fo) v = params[boff[l] - (long)fi * fo + (long)k * fo + n];
     } else {
         j -= FI_WT;
         const int l = j < 3L * FI_W * FI_W ? 1 + (int)(j / (FI_W * FI_W)) : FI_L - 1;
         j -= (l - 1L) * FI_W * FI_W;
         const int fo = l == FI_L - 1 ? FI_OUT : FI_W, ld = l == FI_L - 1 ? 16 : FI_W;
-        const int k = (int)(j / ld), n = (int)(j % ld);
+        int k, n;
+        fi_frag((int)j, ld, k, n);
         if (n < fo) v = params[boff[l] - (long)FI_W * fo + (long)k * fo + n];
     }
     w[i] = (__bf16)v;
@@ -428,7 +442,9 @@ struct TrainBufs {
 constexpr int FI_NB = 4 * FI_W + FI_OUT;  // bias parameters
 __device__ __forceinline__ long fi_a(int l, long ld) { return l == 0 ? 0 : (FI_IN + (l - 1L) * FI_W) * ld; }
 // D[feature][row] for this wave's 64 features of the block's 32 rows; four k
-// steps of weight fragments are in flight ahead of the products
+// steps of weight fragments are in flight ahead of the products.  The chunks stay
+// a loop: unrolled, with the fragments' addresses spelled out, the kernel of 8,192
+// rows takes 61 us, as a loop 36 (51 unrolled with row-by-row weights).
 template <int KIN>
 __device__ __forceinline__ void ft_layer(const __bf16* __restrict__ W, const __bf16 (*H)[FI_LDS], int f0, int lane,
                                          floatx16 (&acc)[2])
@@ -437,7 +453,7 @@ __device__ __forceinline__ void ft_layer(const __bf16* __restrict__ W, const __b
     const __bf16* wp[2];
 #pragma unroll
     for (int f = 0; f < 2; f++) {
-        wp[f] = W + (long)(f0 + f * 32 + (lane & 31)) * KIN + (lane >> 5) * 8;
+        wp[f] = W + (long)(f0 / 32 + f) * 32 * KIN + lane * 8;
 #pragma unroll
         for (int j = 0; j < 16; j++) acc[f][j] = 0.f;
     }
@@ -445,14 +461,14 @@ __device__ __forceinline__ void ft_layer(const __bf16* __restrict__ W, const __b
 #pragma unroll
     for (int f = 0; f < 2; f++)
 #pragma unroll
-        for (int c = 0; c < CH; c++) a[f][c] = *(const bf16x8*)(wp[f] + 16 * c);
-#pragma unroll
+        for (int c = 0; c < CH; c++) a[f][c] = *(const bf16x8*)(wp[f] + 32 * (16 * c));
+#pragma unroll 1
     for (int k0 = 0; k0 < KIN; k0 += 16 * CH) {
         if (k0 + 16 * CH < KIN)
 #pragma unroll
             for (int f = 0; f < 2; f++)
 #pragma unroll
-                for (int c = 0; c < CH; c++) an[f][c] = *(const bf16x8*)(wp[f] + k0 + 16 * (CH + c));
+                for (int c = 0; c < CH; c++) an[f][c] = *(const bf16x8*)(wp[f] + 32 * (k0 + 16 * (CH + c)));
 #pragma unroll
         for (int c = 0; c < CH; c++) {
             const bf16x8 b = *(const bf16x8*)&H[lane & 31][k0 + 16 * c + (lane >> 5) * 8];
