@@ -430,7 +430,7 @@ __global__ void k_pack_weights(const float* __restrict__ params, const long* __r
 //  - k_mlp_sum: the slices' and the blocks' sums.
 // Layer by layer, with FP32 activations in HBM and a column sum of 8,192 rows
 // in four workgroups (385 us a layer), loss and gradient of 8,192 rows took
-// 3.0 ms of kernels; like this 85 us.
+// 3.0 ms of kernels; like this 73 us.
 // ---------------------------------------------------------------------------
 struct TrainBufs {
     __bf16* A;      // A_0 [16][ld], then A_1 .. A_4 [256][ld]
