@@ -910,5 +910,27 @@ FI bool seg_tri(v3 P, v3 Q, v3 A, v3 B, v3 C)
     double u = dot(E2, DAO) * invdet, v = -dot(E1, DAO) * invdet, t = dot(AO, N) * invdet;
     return det >= 1e-12 && t >= 0.0 && u >= 0.0 && v >= 0.0 && (u + v) <= 1.0 && t <= RLen;
 }
+// True when seg_tri accepts no segment in the box slo..shi with a triangle in
+// the box tlo..thi (boxes in single precision that hold the double ones), so the
+// pair need not be tested.  Boxes that are apart are not enough: seg_tri divides
+// by a determinant as small as 1e-12, and for nearly coplanar pairs with edges of
+// some 100 units and more (the determinant grows with their square) its rounding
+// error alone passes the test.  With the triangle's extent e, |P - A| <= a along
+// every axis and unit roundoff w = 2^-53, the errors of the determinant and of
+// the three numerators are at most 21 w e^2, 36 w a e, 36 w a e and 36 w a e^2, so
+// by Cramer's rule the two accepted points are at most 129 w e^2 a / 1e-12 =
+// 0.0144 e^2 a apart along an axis, plus a few w (a + e) for the rest.
+FI bool seg_tri_apart(const float* slo, const float* shi, const float* tlo, const float* thi)
+{
+    float gap = 0.0f, e = 0.0f, a = 0.0f;
+    for (int d = 0; d < 3; d++) {
+        const float g = fmaxf(fmaxf(slo[d] - thi[d], tlo[d] - shi[d]), 0.0f);
+        const float ext = thi[d] - tlo[d];
+        gap = fmaxf(gap, g);
+        e = fmaxf(e, ext);
+        a = fmaxf(a, ext + (shi[d] - slo[d]) + g);
+    }
+    return gap > a * (0.02f * e * e + 1e-12f);
+}
 
 }  // namespace fipc
