@@ -504,6 +504,18 @@ __device__ __forceinline__ void ft_store(const float (&v)[2][16], __bf16 (*H)[FI
             *(uint2*)&H[lane & 31][m] = pk;
         }
 }
+// The last block's rows past n are zeros in every layer and gradient: what the
+// biases alone give there may overflow though no row does, and its product with a
+// zero gradient would be NaN.  In a branch of that block: 64 selects a layer in
+// every block cost 2 us of 8,192 rows' 177.
+__device__ __forceinline__ void ft_mask(float (&v)[2][16], bool row, bool partial)
+{
+    if (partial)
+#pragma unroll
+        for (int f = 0; f < 2; f++)
+#pragma unroll
+            for (int j = 0; j < 16; j++) v[f][j] = row ? v[f][j] : 0.f;
+}
 // column sums over the block's 32 rows: each step hands half of the values to the
 // lane across, so 31 exchanges reduce 32 values; lane l % 32 ends with value l % 32
 template <int N>
@@ -561,6 +573,7 @@ k_mlp_fwdbwd(int n, const float* __restrict__ X, const float* __restrict__ T, co
                 z[l][f][j] = zz;
                 v[f][j] = zz * sigm(zz);
             }
+        ft_mask(v, r0 + (lane & 31) < n, r0 + 32 > n);
         __syncthreads();  // every wave has read this layer's input
         ft_store(v, H, tb.A + fi_a(l + 1, ld), ld, r0, f0, lane);
         __syncthreads();
@@ -619,6 +632,7 @@ k_mlp_fwdbwd(int n, const float* __restrict__ X, const float* __restrict__ T, co
                 const float zz = z[l - 1][f][j], s = sigm(zz);
                 v[f][j] = acc[f][j] * (s * (1.f + zz * (1.f - s)));
             }
+        ft_mask(v, r0 + (lane & 31) < n, r0 + 32 > n);
         __syncthreads();  // every wave has read G_l
         ft_store(v, H, tb.G + (l - 1L) * FI_W * ld, ld, r0, f0, lane);
         ft_colsum(v, bias + (l - 1) * FI_W, f0, lane);

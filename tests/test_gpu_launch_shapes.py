@@ -172,6 +172,35 @@ def test_network_gradient_over_row_remainders(rows):
     net.close()
 
 
+@pytest.mark.parametrize("rows", [1, 2, 4, 8, 16, 64])
+def test_network_gradient_ignores_the_rows_past_the_last(rows):
+    """The rows that fill up a block of 32 add nothing, also where the biases alone
+    overflow: here a row of zeros gives 2^66 in the first layer and infinity in the
+    second, while the rows themselves give zero.  All rows are alike, so the mean's
+    gradient is that of one full block; with powers of two every product scales
+    exactly, which leaves the rounding of FP32 sums of up to 64 equal terms."""
+    from fastipc_amd.warmstart import WarmStartMLP
+    net = WarmStartMLP(seed=1)
+    big, w = 2.0 ** 66, net.params()
+    W0 = w[:16 * 256].reshape(16, 256)
+    W0[:], W0[0] = 0, -big
+    w[16 * 256:17 * 256] = big
+    w[17 * 256:17 * 256 + 256 * 256] = big
+    net.set_params(w)
+
+    def grad(n):
+        X = np.zeros((n, 16), np.float32)
+        X[:, 0] = 1
+        return net.grad(X, np.ones((n, 3), np.float32))
+
+    loss, g = grad(rows)
+    loss32, g32 = grad(32)
+    assert np.isfinite(g).all() and np.abs(g32).max() > 0
+    assert abs(loss - loss32) <= 64 * 2.0 ** -24 * loss32
+    assert np.linalg.norm(g - g32) <= 64 * 2.0 ** -24 * np.linalg.norm(g32)
+    net.close()
+
+
 @pytest.mark.parametrize("kind", [0, 1])
 def test_batch_ccd_does_not_depend_on_the_number_of_pairs(kind):
     """A pair's time is the same bits alone and in full and partial blocks of 64."""
