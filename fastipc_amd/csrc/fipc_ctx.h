@@ -22,6 +22,18 @@
         }                                                                             \
     } while (0)
 
+// The stop word of a solve's iterations.  The host queues iterations ahead of its
+// checks; the launches of iteration it leave at their start when pcg_past.  The
+// update of iteration it tests the residual of the one before, and its block 0
+// stores pcg_stop(it) when that passes, while other waves of the same launch may
+// still be about to read the word: for them it must say stay, whichever value
+// they read, or some waves of a block would leave and the others sum what those
+// never wrote.  So the launch that stores it is not past it, every later one is.
+constexpr int PCG_RUNNING = 0x7fffffff;  // not stopped
+constexpr int PCG_AT_START = -1;         // the residual at the start passes: no iteration runs
+FI bool pcg_past(int it, int stop) { return it > stop; }
+FI int pcg_stop(int it) { return it; }
+
 #define STCHK(expr)                       \
     do {                                  \
         int _st = (expr);                 \

@@ -1035,7 +1035,7 @@ k_spmv(int nv, const int* __restrict__ rowptr, const int* __restrict__ col, cons
 {
     // the test that ends the launches queued past convergence is loaded with
     // the first row bounds (slot bounds), not ahead of them
-    const int last = state ? state[0] : 0x7fffffff;
+    const int stop = state ? state[0] : PCG_RUNNING;
     double pq = 0.0;
     if ((int)blockIdx.x >= nl_c) {
         // the row groups are split into 8 contiguous ranges, one per XCD
@@ -1057,7 +1057,7 @@ k_spmv(int nv, const int* __restrict__ rowptr, const int* __restrict__ col, cons
         bool live = row < nv && g0 < g1;
         int nu0 = live ? rowptr[row] : 0, nu1 = live ? rowptr[row + 1] : 0;
         int nl0 = live ? lptr[row] : 0, nl1 = live ? lptr[row + 1] : 0;
-        if (it > last) return;
+        if (pcg_past(it, stop)) return;
         for (int g = g0; g < g1; g += nbx) {
             row = g * SPMV_ROWS + rsub;
             int u0 = nu0, l0 = nl0;
@@ -1115,7 +1115,7 @@ k_spmv(int nv, const int* __restrict__ rowptr, const int* __restrict__ col, cons
         const int u = gid / CV_G, l = gid % CV_G;
         const int n = cs.count[0];
         const int e0 = u < cs.nslots ? cs.ptr[u] : 0, e1 = u < cs.nslots ? cs.ptr[u + 1] : 0;
-        if (it > last) return;
+        if (pcg_past(it, stop)) return;
         const bool live = u < n;
         double sv[3] = {0.0, 0.0, 0.0};
         if (live) contact_vertex_spmv<V>(cs, p, e0 + l, e1, sv);
@@ -1195,7 +1195,7 @@ __global__ void k_pcg_init(int nv, const double* b, const double* q, const doubl
 // scal[0|1] = rz from partials.  First start: scal[2|3] = |r0|^2, the
 // reference norm of the relative tolerance.  Restart (refinement): the
 // partials hold |r|^2 of the recomputed FP64 residual, kept in scal[4];
-// state[0] = -1 when that residual already meets the tolerance.
+// state[0] = PCG_AT_START when that residual already meets the tolerance.
 __global__ void k_pcg_scalars(const double* part_rz, const double* part_bb, int n, double* scal, int* state,
                               int restart, double tol2)
 {
@@ -1205,10 +1205,10 @@ __global__ void k_pcg_scalars(const double* part_rz, const double* part_bb, int 
         scal[0] = rz; scal[1] = rz;
         if (!restart) {
             scal[2] = bb; scal[3] = bb; scal[4] = bb;
-            state[0] = bb == 0.0 ? -1 : 0x7fffffff;  // done_at
+            state[0] = bb == 0.0 ? PCG_AT_START : PCG_RUNNING;
         } else {
             scal[4] = bb;
-            state[0] = (bb <= tol2 * scal[2] || !(bb == bb)) ? -1 : 0x7fffffff;
+            state[0] = (bb <= tol2 * scal[2] || !(bb == bb)) ? PCG_AT_START : PCG_RUNNING;
         }
         state[1] = 0;
     }
@@ -1219,17 +1219,16 @@ __global__ void k_pcg_retest(const double* scal, int* state, double tol2)
 {
     if (threadIdx.x == 0) {
         double bb = scal[4];
-        state[0] = (bb <= tol2 * scal[2] || !(bb == bb)) ? -1 : 0x7fffffff;
+        state[0] = (bb <= tol2 * scal[2] || !(bb == bb)) ? PCG_AT_START : PCG_RUNNING;
         state[1] = 0;
     }
 }
 // scal[0] = r.z of a round's start, scal[2] = |r0|^2, scal[4] = |r|^2 of
 // the last tested residual, scal[5] = u.A u of the last iteration,
 // scal[6|7] and scal[8|9] = gamma and alpha of an iteration (by parity);
-// state[0] = iteration at which the test passed (done_at), state[1] =
-// iterations run.  The update kernel runs a grid-stride loop over vertices on
-// at most PCG_MAXB blocks, so the partials that the next kernel reduces stay
-// few.
+// state[0] = the stop word (fipc_ctx.h), state[1] = iterations run.  The update
+// kernel runs a grid-stride loop over vertices on at most PCG_MAXB blocks, so the
+// partials that the next kernel reduces stay few.
 // the FP32 iterations stop at this fraction of the tolerance, so that the
 // FP64 residual that follows usually meets it
 #ifndef PCG_FP32_INNER
@@ -1258,8 +1257,8 @@ static inline int pcg_grid(int nv) { return std::min(nblk(nv), PCG_MAXB); }
 // solution (FP64 rounds) or, in the FP32 rounds, the round's correction in
 // FP32, which k_pcg_flush adds to the FP64 solution when the round ends.  The test of
 // an iteration's residual runs at the start of the next one (every block
-// decides it from the same partials; block 0 records it): on success
-// done_at = it - 1 and nothing more is written.  gamma and alpha of an
+// decides it from the same partials; block 0 sets the stop word): on success
+// nothing more is written.  gamma and alpha of an
 // iteration are kept by parity in scal[6 + (it & 1)] and scal[8 + (it & 1)],
 // so no block reads a value another block of the same launch writes.  One
 // launch replaces the two update kernels of the textbook form (whose second
@@ -1310,7 +1309,7 @@ __global__ void __launch_bounds__(TPB) k_pcg_cg(int nv, double* scal, const unsi
                                                 int* state, int it, double tol2)
 {
     const int cur = it & 1, prv = cur ^ 1;
-    const int last = state[0];
+    const int stop = state[0];
     const double* pg = part_g + 2 * PCG_MAXB * prv;
     double sd = 0.0, sg = 0.0, sr = 0.0;
     // the product's partials: all, or (ncv set) those of the contact blocks that
@@ -1333,7 +1332,7 @@ __global__ void __launch_bounds__(TPB) k_pcg_cg(int nv, double* scal, const unsi
     int i = blockIdx.x * TPB + threadIdx.x;
     CgVertex<V, M> a;
     if (i < nv) cg_load(a, i, it == 0, mask, Minv, u, w, p, s, x, r);
-    if (it > last) return;
+    if (pcg_past(it, stop)) return;
     if (ncv) {
         if ((int)threadIdx.x < used) sd += c0;
         for (int j = threadIdx.x + TPB; j < used; j += TPB) sd += part_uw[j];
@@ -1357,7 +1356,7 @@ __global__ void __launch_bounds__(TPB) k_pcg_cg(int nv, double* scal, const unsi
         rr = res0;
     } else if (rr <= tol2 * rr0 || !(rr == rr)) {
         if (blockIdx.x == 0 && threadIdx.x == 0) {
-            state[0] = it - 1;
+            state[0] = pcg_stop(it);
             state[1] = it;
             scal[4] = rr;
         }
@@ -1423,13 +1422,13 @@ __global__ void __launch_bounds__(TPB) k_pcg_cg(int nv, double* scal, const unsi
 // before the next iteration could run it
 __global__ void k_pcg_cg_last(double* scal, const double* part_g, int npg, int* state, int it, double tol2)
 {
-    if (it > state[0]) return;
+    if (pcg_past(it, state[0])) return;
     const int prv = (it & 1) ^ 1;
     double gamma, rr;
     reduce_partials2(part_g + 2 * PCG_MAXB * prv, part_g + 2 * PCG_MAXB * prv + PCG_MAXB, npg, gamma, rr);
     if (threadIdx.x == 0) {
         scal[4] = rr;
-        if (rr <= tol2 * scal[2] || !(rr == rr)) state[0] = it - 1;
+        if (rr <= tol2 * scal[2] || !(rr == rr)) state[0] = pcg_stop(it);
     }
 }
 
@@ -2359,7 +2358,7 @@ static int pcg_round(fipc_ctx* c, int prec, const M* Minv, V* r, V* z, V* p, V* 
     // the iterations' x: the FP64 solution, or the FP32 round's correction
     V* xs = sizeof(V) == 4 ? (V*)(void*)c->dxf.p : (V*)(void*)c->sol.p;
     int it = 0;
-    state[0] = 0x7fffffff;
+    state[0] = PCG_RUNNING;
     state[1] = 0;
     *init_only = false;
     *cert_stop = false;
@@ -2383,7 +2382,7 @@ static int pcg_round(fipc_ctx* c, int prec, const M* Minv, V* r, V* z, V* p, V* 
             // the recomputed residual may already meet the tolerance
             STCHK(d2h_async(c, state, c->pcg_state.p, 8));
             STCHK(d2h_wait(c));
-            if (state[0] == -1) {
+            if (state[0] == PCG_AT_START) {
                 *init_only = true;
                 return FIPC_OK;
             }
@@ -2397,7 +2396,7 @@ static int pcg_round(fipc_ctx* c, int prec, const M* Minv, V* r, V* z, V* p, V* 
         STCHK(cert_check(c, &ok));
         if (ok) {
             c->cert_hit = true;
-            state[0] = -1;
+            state[0] = PCG_AT_START;
             return FIPC_OK;
         }
         if (it == 0) c->cert_fail++;
@@ -2429,7 +2428,7 @@ static int pcg_round(fipc_ctx* c, int prec, const M* Minv, V* r, V* z, V* p, V* 
         STCHK(d2h_async(c, state, c->pcg_state.p, 8));
         if (cert) STCHK(d2h_async(c, &rr, c->scal.p + 4, 8));
         STCHK(d2h_wait(c));
-        if (state[0] != 0x7fffffff) break;
+        if (state[0] != PCG_RUNNING) break;
         // the recursive residual suggests the certificate holds: end the
         // round, whose successor's restart checks it with the FP64 residual
         // (after a failed check, only at half the bound)
@@ -2456,7 +2455,7 @@ static int pcg_round(fipc_ctx* c, int prec, const M* Minv, V* r, V* z, V* p, V* 
         HIPCHK(hipGetLastError());
     }
     // the budget ran out: the last iteration's residual is tested here
-    if (state[0] == 0x7fffffff && it > 0 && !*cert_stop) {
+    if (state[0] == PCG_RUNNING && it > 0 && !*cert_stop) {
         k_pcg_cg_last<<<1, TPB, 0, c->s>>>(c->scal.p, c->part_g.p, nu, c->pcg_state.p, it, tol_it);
         HIPCHK(hipGetLastError());
         STCHK(d2h_async(c, state, c->pcg_state.p, 8));
@@ -2525,24 +2524,24 @@ static int solve_rounds(fipc_ctx* c, int first_round, double tol, int maxit, int
         else
             STCHK((pcg_round<double, double>(c, prec, c->Minv.p, c->r.p, c->z.p, c->pp.p, c->q.p, round, budget,
                                              tol2, hint, state, ru, &init_only, &cert_stop)));
-        if (state[0] == -1 && round > 0) { converged = true; break; }
-        int ran = state[0] == -1 ? 0 : state[1];
+        if (state[0] == PCG_AT_START && round > 0) { converged = true; break; }
+        int ran = state[0] == PCG_AT_START ? 0 : state[1];
         total += ran;
         if (round == 0 && ran > 0) c->pcg_hint = ran;
         if (round == first_round && first_round > 0 && ran > 0 && !cert_stop) c->refine_hint = ran;
         if (cert_stop) continue;                  // the next round's restart checks the certificate
-        if (state[0] == 0x7fffffff) break;        // iteration budget spent
-        if (prec != 1 || state[0] == -1) { converged = true; break; }
+        if (state[0] == PCG_RUNNING) break;        // iteration budget spent
+        if (prec != 1 || state[0] == PCG_AT_START) { converged = true; break; }
         // FP32 iterations converged: the next round checks the FP64 residual
     }
     // refinement rounds exhausted after a converged FP32 round: the FP64
     // residual of its result decides (one more product, no iterations); the
     // solve is reported as not converged when it misses the tolerance
-    if (!converged && state[0] != 0x7fffffff) {
+    if (!converged && state[0] != PCG_RUNNING) {
         int chk[2] = {0, 0};
         STCHK((pcg_round<float, float>(c, prec, c->Minvf.p, c->rf.p, c->zf.p, c->pf.p, c->qf.p,
                                        first_round + rounds, 0, tol2, 0, chk, false, &init_only, &cert_stop)));
-        converged = chk[0] == -1;
+        converged = chk[0] == PCG_AT_START;
     }
     // a solve that ended on a restart whose FP64 residual met the tolerance
     // leaves that restart for a continuation
