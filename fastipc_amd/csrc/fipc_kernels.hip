@@ -1938,6 +1938,8 @@ extern "C" int fipc_upload_mesh(fipc_ctx* c, int nv, const double* x0, const dou
 extern "C" int fipc_set_params(fipc_ctx* c, double dt, double dHat, double kappa, double inv_dx, double gravity)
 {
     if (!c || !(dt > 0) || !(dHat > 0) || !(inv_dx > 0)) return FIPC_ERR_ARG;
+    // grids of another cell size are not reused
+    if (inv_dx != c->inv_dx) c->grid[0].reusable = c->grid[1].reusable = false;
     c->dt = dt; c->dHat = dHat; c->dHat2 = dHat * dHat; c->kappa = kappa; c->inv_dx = inv_dx; c->gravity = gravity;
     c->e_ok = false;
     return FIPC_OK;

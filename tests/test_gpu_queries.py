@@ -93,3 +93,30 @@ def test_swept_candidates_and_searches_along_the_step(n, copies, spread, offset)
         sim.find_constraints()
         assert tuple(sim.search_counts()) == _near(sim.x, sc, dhat), alpha
     sim.close()
+
+
+@pytest.mark.parametrize("factor", [0.3, 3.0])
+def test_cell_size_changed_between_searches(factor):
+    """Grids of the former cell size are not reused at the same positions."""
+    sc, rng = _crowd(3, 2, 0.2, 0.0)
+    sim = NewtonIPC(sc)
+    s = sim.setup
+    x = sc.x + rng.normal(0, 0.01, sc.x.shape)
+    sim.set_state(x, np.zeros_like(x))
+    sim.set_vector(1, rng.normal(0, 0.03, sc.x.shape))
+    sim.save_xPrev()
+    sim.search_stats(True)
+    want = _near(x, sc, s.dHat)
+    for inv_dx in (s.inv_dx, factor * s.inv_dx):
+        _lib.call("fipc_set_params", sim.ctx, s.dt, s.dHat, s.kappa, inv_dx, s.gravity)
+        sim.find_constraints()
+        assert tuple(sim.search_counts()) == want
+    # the same with the step bound's grids of swept boxes
+    sim.compute_intersection_free_step_size()
+    sim.apply_sol(1.0)
+    want = _near(sim.x, sc, s.dHat)
+    for inv_dx in (factor * s.inv_dx, s.inv_dx):
+        _lib.call("fipc_set_params", sim.ctx, s.dt, s.dHat, s.kappa, inv_dx, s.gravity)
+        sim.find_constraints()
+        assert tuple(sim.search_counts()) == want
+    sim.close()
