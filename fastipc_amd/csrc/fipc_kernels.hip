@@ -1996,6 +1996,7 @@ extern "C" int fipc_set_vector(fipc_ctx* c, int which, const double* in)
     if (!d || !in) return FIPC_ERR_ARG;
     HIPCHK(hipMemcpyAsync(d->p, in, (size_t)c->nv * 24, hipMemcpyHostToDevice, c->s));
     if (d == &c->x) c->x_version++;
+    if (d == &c->xprev) c->xprev_of = 0;  // no x that a grid was built at
     if (d != &c->sol) c->sys_version++;   // a continued solve needs the system it solved
     c->restart_ready = false;
     if (d == &c->sol) c->sol_version++;

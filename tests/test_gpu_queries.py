@@ -120,3 +120,21 @@ def test_cell_size_changed_between_searches(factor):
         sim.find_constraints()
         assert tuple(sim.search_counts()) == want
     sim.close()
+
+
+def test_previous_positions_set_before_a_step():
+    """A step from positions that the caller set is not on the segment that the
+    step bound's grids sweep."""
+    sc, rng = _crowd(3, 2, 0.2, 0.0)
+    sim = NewtonIPC(sc)
+    x = sc.x + rng.normal(0, 0.01, sc.x.shape)
+    sim.set_state(x, np.zeros_like(x))
+    sim.set_vector(1, rng.normal(0, 0.03, sc.x.shape))
+    sim.save_xPrev()
+    sim.compute_intersection_free_step_size()
+    sim.set_vector(5, x + rng.normal(0, 0.2, sc.x.shape))
+    sim.apply_sol(0.5)
+    sim.search_stats(True)
+    sim.find_constraints()
+    assert tuple(sim.search_counts()) == _near(sim.x, sc, sim.setup.dHat)
+    sim.close()
