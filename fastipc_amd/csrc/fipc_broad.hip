@@ -5,10 +5,11 @@
 // Grid: every inserted item is entered in each cell its box overlaps
 // (cell size = 1 / inv_dx, as the reference's hash).  Entries are grouped by
 // a hashed bucket; each entry keeps its exact 63-bit cell key and three bits
-// telling whether the cell is the item's lowest cell along x, y, z.  A query
-// runs one thread per (query box, cell) pair, so huge boxes do not serialise
-// a wave, and accepts an entry only in the first cell common to both boxes,
-// so every pair is tested exactly once.  Builds and queries size their
+// telling whether the cell is the item's lowest cell along x, y, z.  A wave of
+// a query takes up to 64 (query box, cell) pairs and runs over their cells'
+// entries laid end to end, so neither huge boxes nor crowded cells serialise
+// it; an entry is accepted only in the first cell common to both boxes, so
+// every pair is tested exactly once.  Builds and queries size their
 // buffers from capacities and never wait for the host; each operation
 // synchronises once at its end and is redone when a capacity was exceeded.
 #include <hip/hip_runtime.h>
@@ -319,7 +320,7 @@ struct QueryWave {
 // every entry cost a chain of dependent loads (cell, item, vertex numbers,
 // vertices) in a wave as long as its longest bucket.  Like that, and like this:
 // edge-edge CCD candidates on 200 cubes of 8^3 (176,400 surface edges) 332 and
-// 190 us, collision test 196 and 127; on the 1M-tet slab 84 and 70, 68 and 53;
+// 190 us, collision test 196 and 114; on the 1M-tet slab 84 and 70, 68 and 49;
 // edge-edge search on two cubes of 10^3 45 and 19 us.  Registers set the waves
 // in flight (Visit::waves per SIMD; one more spills and takes 1.3 to 2 times as
 // long).

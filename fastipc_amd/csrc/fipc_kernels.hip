@@ -1270,7 +1270,7 @@ static inline int pcg_grid(int nv) { return std::min(nblk(nv), PCG_MAXB); }
 // pass, each in its own order) and the thread's first vertex.  In the order of
 // use, with a barrier pair per sum, it took 7.0 us on 2,008 vertices and 18.0 on
 // 110,600 in FP64, 6.5 on 24,695 and 14.5 on 200,016 in FP32; like this 4.6,
-// 14.0, 4.9 and 10.6 (200,016 vertices: 3.4 TB/s).
+// 14.0, 4.9 and 10.6 (200,016 vertices, 169 bytes each: 3.2 TB/s).
 // mask: bit 0 Dirichlet vertex, bit 1 contact vertex (whose product has a
 // contact part in qc; qc is read nowhere else).
 template <class V, class M>

@@ -430,7 +430,8 @@ __global__ void k_pack_weights(const float* __restrict__ params, const long* __r
 //  - k_mlp_sum: the slices' and the blocks' sums.
 // Layer by layer, with FP32 activations in HBM and a column sum of 8,192 rows
 // in four workgroups (385 us a layer), loss and gradient of 8,192 rows took
-// 3.0 ms of kernels; like this 73 us.
+// 3.0 ms of kernels; like this 69 us (35 + 28 + 6; the packing, once the
+// parameters changed, 8 more).
 // ---------------------------------------------------------------------------
 struct TrainBufs {
     __bf16* A;      // A_0 [16][ld], then A_1 .. A_4 [256][ld]
@@ -818,8 +819,9 @@ static int mlp_loss_parts(const fipc_mlp* m, int n) { return m->fused ? (n + 31)
 static int mlp_backward_fused(fipc_mlp* m, hipStream_t s, int n, const float* X, const float* T)
 {
     const int nb = (n + 31) / 32;
-    // rows per slice of the weight gradients: at most 32 slices, of at least 256
-    // rows (a multiple of the four waves' 64)
+    // the weight gradients' row slices, at most 32: one below 1,024 rows, then of
+    // at least 512, rounded up to the four waves' 64 rows.  So the last ones may be
+    // short or empty (16,416 rows: 28 of 576, one of 288, three that store zeros)
     const long ld = 32L * nb;
     const int S = (int)std::max(1L, std::min(32L, ld / 512));
     const int slice = (int)((ld + 64L * S - 1) / (64L * S)) * 64;
